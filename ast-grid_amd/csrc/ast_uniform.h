@@ -81,11 +81,12 @@ private:
     hipStream_t stream_;
     AstGeom g_;
     PcgDevice pcg_;
-    DevBuf open_, tid_, tnode_, flag_, scan_, mac_[3], tilt_, len_, rs_, col_, tmp_, bmax_, keys_;
+    DevBuf open_, tid_, tnode_, flag_, scan_, mac_[3], tilt_, len_, rs_, col_, tmp_, bmax_, keys_, coord_;
     BlockOrderDevice blk_;
     std::unique_ptr<PcgDevice> pcgBlk_;  // the block-colour copy of the system
     int n_ = 0;
     long long nnz_ = 0;
+    bool coords_ = false;  // the rows have packed positions (coord_)
     bool patternReady_ = false;
     bool blkReady_ = false;
     bool solved_ = false;

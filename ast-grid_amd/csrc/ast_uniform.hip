@@ -299,6 +299,26 @@ __global__ void k_ast_block_keys(AstGeom g, int n, const int* tnode, int B, int*
     keys[r] = colour * (nbx * nby * nbz) + bx + nbx * (by + nby * bz);
 }
 
+// Position of every row on the doubled grid (cell centres odd), packed as
+// PcgDevice::setCoords takes it.
+template <int D>
+__global__ void k_ast_coords(AstGeom g, int n, const int* tnode, unsigned long long* coord) {
+    const int r = blockIdx.x * BS + threadIdx.x;
+    if (r >= n) return;
+    unsigned long long x, y, z = 0;
+    if (r < g.nc) {
+        x = 2 * (r % g.res[0]) + 1;
+        y = 2 * ((r / g.res[0]) % g.res[1]) + 1;
+        if (D == 3) z = 2 * (r / (g.res[0] * g.res[1])) + 1;
+    } else {
+        const long long t = tnode[r - g.nc], tx = g.res[0] + 1, ty = g.res[1] + 1;
+        x = 2 * (t % tx);
+        y = 2 * ((t / tx) % ty);
+        if (D == 3) z = 2 * (t / (tx * ty));
+    }
+    coord[r] = z << 36 | y << 18 | x;
+}
+
 // correctVelocityByPressure, tilt part (ast_solver.h:286-296).
 template <int D>
 __global__ void k_ast_correct_tilt(AstGeom g, int nOpen, const int* tnode, const double* p, double* tu, double dt,
@@ -504,6 +524,19 @@ int AstUniform::ensurePattern(std::string& err) {
                                                            nullptr, 0.0);
     HIPCHK(hipGetLastError());
     pcg_.setMergeLevels(astRefMerge(g_.d));
+    // rows' positions for the tiled sweeps (18 bits per axis; beyond, none)
+    coords_ = std::max({g_.res[0], g_.res[1], g_.d == 3 ? g_.res[2] : 0}) < (1 << 17);
+    const int ext[3] = {2 * g_.res[0] + 1, 2 * g_.res[1] + 1, g_.d == 3 ? 2 * g_.res[2] + 1 : 1};
+    if (coords_) {
+        HIPCHK(coord_.alloc((size_t)n * 8));
+        if (g_.d == 2)
+            k_ast_coords<2><<<nblk(n), BS, 0, stream_>>>(g_, n, tnode_.as<int>(), coord_.as<unsigned long long>());
+        else
+            k_ast_coords<3><<<nblk(n), BS, 0, stream_>>>(g_, n, tnode_.as<int>(), coord_.as<unsigned long long>());
+        if (int rc2 = pcg_.setCoordsDevice(n, coord_.as<unsigned long long>(), nullptr, ext, err)) return rc2;
+    } else {
+        (void)pcg_.setCoords(0, nullptr, nullptr, err);
+    }
     int rc = pcg_.setPatternDevice(n, nnz, rs_.as<int>(), col_.as<int>(), err);
     if (rc) return rc;
     n_ = n;
@@ -554,6 +587,13 @@ int AstUniform::ensureBlockOrder(std::string& err) {
     if (rc) return rc;
     if (!pcgBlk_) pcgBlk_.reset(new PcgDevice(stream_));
     pcgBlk_->setMergeLevels(astMerge(n_));
+    pcgBlk_->setTileFp32(true);
+    if (coords_) {
+        const int ext[3] = {2 * g_.res[0] + 1, 2 * g_.res[1] + 1, g_.d == 3 ? 2 * g_.res[2] + 1 : 1};
+        if ((rc = pcgBlk_->setCoordsDevice(n_, pcg_.devCoords(), blk_.perm.as<int>(), ext, err))) return rc;
+    } else {
+        (void)pcgBlk_->setCoords(0, nullptr, nullptr, err);
+    }
     rc = pcgBlk_->setPatternDevice(n_, nnz_, blk_.rowstart.as<int>(), blk_.col.as<int>(), err);
     if (rc) return rc;
     blkReady_ = true;

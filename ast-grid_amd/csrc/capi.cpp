@@ -36,6 +36,7 @@ struct astg_ctx {
     std::unique_ptr<astg::PcgDevice> pcgBlk;              // the same system in block-colour order (reorder.h)
     astg::BlockOrderDevice blk;  // permutation and permuted pattern, device-built
     bool blkReady = false;
+    int coordExt[3] = {0, 0, 0};  // extents of the rows' positions (rowCoords)
     bool factoredBlk = false;  // the last factorisation was of the block-colour copy
     std::unique_ptr<astg::ProjectDevice> proj;
     std::unique_ptr<astg::AdvectDevice> adv;              // post-projection step and advection
@@ -77,6 +78,14 @@ int needDevice(astg_ctx* c) {
     return ASTG_OK;
 }
 
+// The projection system's pattern, with the rows' positions.
+int setProjectionPattern(astg_ctx* c) {
+    std::vector<unsigned long long> coord;
+    astg::rowCoords(*c->tree, c->num, coord, c->coordExt);
+    if (int rc = c->pcg->setCoords(c->tables.n, coord.data(), c->coordExt, c->err)) return rc;
+    return c->pcg->setPattern(c->tables.n, c->tables.rowstart.data(), c->tables.col.data(), c->err);
+}
+
 int ensureTables(astg_ctx* c) {
     if (!c->tree) return fail(c, ASTG_ERR_STATE, "no topology set");
     if (!c->tablesReady) {
@@ -105,8 +114,7 @@ int ensureTables(astg_ctx* c) {
         if (!c->adv) c->adv.reset(new astg::AdvectDevice(c->stream));
         rc = c->adv->upload(*c->tree, c->tables, false, c->err);
         if (rc) return rc;
-        rc = c->pcg->setPattern(c->tables.n, c->tables.rowstart.data(), c->tables.col.data(), c->err);
-        if (rc) return rc;
+        if ((rc = setProjectionPattern(c))) return rc;
         // fields, and the advection's output buffers, start at zero
         const size_t G = c->tables.G;
         std::vector<double> z((size_t)8 * G, 0.0);
@@ -161,7 +169,7 @@ int retopologizeSteps(astg_ctx* c) {
     rc = c->adv->upload(*c->tree, c->tables, true, c->err);
     if (rc) return rc;
     tm.mark("advect upload");
-    rc = c->pcg->setPattern(c->tables.n, c->tables.rowstart.data(), c->tables.col.data(), c->err);
+    rc = setProjectionPattern(c);
     tm.mark("solver pattern");
     long long na1;
     double ma1;
@@ -562,6 +570,9 @@ int ensureBlockOrder(astg_ctx* c) {
     }
     if (!c->pcgBlk) c->pcgBlk.reset(new astg::PcgDevice(c->stream));
     c->pcgBlk->setMergeLevels(blockMerge());
+    c->pcgBlk->setTileFp32(true);
+    if ((rc = c->pcgBlk->setCoordsDevice(n, c->pcg->devCoords(), c->blk.perm.as<int>(), c->coordExt, c->err)))
+        return rc;
     rc = c->pcgBlk->setPatternDevice(n, nnz, c->blk.rowstart.as<int>(), c->blk.col.as<int>(), c->err);
     if (rc) return rc;
     tm.mark("solver pattern");

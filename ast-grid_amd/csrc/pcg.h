@@ -7,10 +7,11 @@
 //     sync-free pass;
 //   * the factorisation is level-synchronous (one launch per level, one row per
 //     lane, left-looking per row with the reference's accumulation order);
-//   * the triangular sweeps are sync-free persistent kernels over merged
-//     stencils (sweep_merge.h): each row publishes its value with an
-//     agent-scope atomic store over a signalling-NaN sentinel that dependants
-//     poll;
+//   * the triangular sweeps run in spatial tiles, one workgroup each, whose
+//     rows' values live in LDS (tile_sweep.h); systems too large for that, and
+//     batches, take sync-free persistent kernels over merged stencils
+//     (sweep_merge.h): each row publishes its value with an agent-scope atomic
+//     store over a signalling-NaN sentinel that dependants poll;
 //   * dots, axpys and the convergence test are fused into the SpMV / update /
 //     sweep kernels with wave64 reductions; scalars stay on the device.
 #pragma once
@@ -23,6 +24,7 @@
 
 #include "../../include/astg.h"
 #include "device_common.h"
+#include "tile_sweep.h"
 
 namespace astg {
 class PhaseTimer;
@@ -90,6 +92,16 @@ struct StencilView {
 struct DevStencil {
     DevBuf start, nr, idx, ustart, upd, coef, coef32;
     long long E = 0;  // entries (r-terms plus y-terms) over all rows
+};
+
+// LDS a tile of the tiled sweeps may take (160 KB per CU less the reductions').
+constexpr size_t kTileLdsBytes = 160 * 1024 - 1024;
+
+// One direction of the tiled sweeps (tile_sweep.h).
+struct DevTile {
+    DevBuf sell, slot, hstart, xstart, xslot, xdest, inbox, coef, coef32;
+    long long E = 0;  // stored entries, padding included
+    int halo = 0;     // halo entries of all tiles
 };
 
 // Per-block partials of the reductions, consumed by the next kernel.
@@ -184,6 +196,17 @@ public:
     // Keep the PCG vectors in row order (the batched form, whose streaming
     // kernels work per system on stacked rows). Takes effect at setPattern.
     void setRowOrder(bool on) { rowOrderForced_ = on; }
+    // Positions of the next pattern's rows, for the tiled sweeps: n packed
+    // coordinates z << 36 | y << 18 | x (host memory), each below ext. Without
+    // them (null, the default) tiles are index ranges.
+    int setCoords(int n, const unsigned long long* coord, const int* ext, std::string& err);
+    // The same from device memory on this object's stream; row i is at
+    // coord[perm[i]] (perm null: coord[i]).
+    int setCoordsDevice(int n, const unsigned long long* coord, const int* perm, const int* ext, std::string& err);
+    const unsigned long long* devCoords() const { return rowCoord_.as<unsigned long long>(); }
+    // Tiles whose values fit the LDS in FP32 only are taken too: for a pattern
+    // whose solves are the mixed form's (an FP64 solve then rebuilds it).
+    void setTileFp32(bool on) { tileFp32_ = on; }
     // Levels per merged sweep group used by the next setPattern (0: default).
     void setMergeLevels(int q) { mergeLevels_ = q; }
     int mergeLevels() const { return merge_; }
@@ -223,7 +246,7 @@ private:
     // symbolic plans (factorisation programs, both merged stencils) built on
     // the device from the uploaded pattern and sweep order (plan_device.hip);
     // the host planners serve when hostPlan_ is set
-    int planDevice(int maxY, std::string& err);
+    int planDevice(int maxY, bool stencils, std::string& err);
     // Sweep-ordered solve: permuted CSR, forward r-term keys as positions
     // (once per pattern); values, pivots and rhs gathered per solve.
     int permuteSetup(std::string& err);
@@ -238,6 +261,24 @@ private:
     template <typename T>
     void launchSpmv(int n, const int* rs, const int* col, const T* A, const T* s, T* q, const Parts& Pt,
                     const double* scal);
+    // Tiled sweeps (tile_sweep.hip): the tiles of the pattern (used false: they
+    // do not fit, the merged sweeps serve), their coefficients, one launch.
+    int tileSetup(bool& used, std::string& err);
+    int dropTiles(std::string& err);
+    bool tilesFit(int slots, int width) const;  // values of `width` bytes: the LDS holds them
+    size_t tileLds(int slots, int width) const;
+    TileView tileView() const;
+    template <typename T>
+    int tileCoef(std::string& err);
+    template <typename T>
+    int launchTile(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm, double tolRel,
+                   int phases, std::string& err);
+    template <typename T>
+    void armSweeps();
+    // One preconditioning z = (L L^T)^-1 r: sweep k of a solve.
+    template <typename T>
+    int precondition(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm, double tolRel,
+                     std::string& err);
     int launchMic(double tau, double ratio, std::string& err);
     int launchMerge(std::string& err);
     int convert32(std::string& err);
@@ -307,6 +348,18 @@ private:
     DevBuf prs_, pcol_, pmap_;              // CSR in sweep order: rowstart, columns as positions, source entry
     DevBuf valP_, invdP_, bP_, xP_;         // values, pivots, rhs and solution in sweep order
     DevBuf permLen_;                        // set-up: row lengths in sweep order
+    // tiled sweeps
+    bool tiled_ = false;                    // the current pattern sweeps in tiles
+    bool noTile_ = false;                   // dropTiles: this set-up takes the merged sweeps
+    bool tileFp32_ = false;                 // setTileFp32
+    bool tileCoef64_ = false;               // FP64 tile coefficients match the factor
+    bool tileLds64_ = false, tileLds32_ = false;  // dynamic LDS limit raised
+    int tileK_ = 0, tileS_ = 0, tileSlots_ = 0;
+    int tileExports_ = 0;                   // longest export list of a tile
+    int coordExt_[3] = {0, 0, 0};           // coordinate extents of rowCoord_ (0: none)
+    DevTile tile_[2];
+    DevBuf rowCoord_, tileStep_;            // row positions; steps
+    DevBuf tileKey_, tileKey2_, tileVal_, tileVal2_, tileOf_, tileCnt_, tileMax_, entryHalo_;  // set-up
     bool batchGraph_ = true;                // batched form: iterations replayed from hipGraphs
     bool coop_ = false;                     // sweeps through the cooperative launch API (ASTG_COOP=1)
     bool spinFailed_ = false;               // a sweep hit its spin limit since the last solve started

@@ -340,43 +340,6 @@ __global__ void __launch_bounds__(BS) k_init(int n, const T* b, X* x, T* r, Part
     if (threadIdx.x == 0) Pt.res[blockIdx.x] = t;
 }
 
-// Forward sweep y = L^-1 r. mode 0 (start of the solve): ||b|| from the
-// partials, tolerance, zero-rhs exit. mode 1 (iteration `it`): the reference's
-// convergence test on the updated residual, before preconditioning. mode 2:
-// no test here (the batched solve tests each system in its own kernel).
-// Returns true when the solve stops here (every block takes the same decision).
-__device__ inline bool fwd_prologue(const Parts& Pt, double* scal, int mode, int it, int maxIt, int norm,
-                                    double tolRel) {
-    double red = norm == ASTG_NORM_INF ? reduce_prev<true>(Pt.res, Pt.gs) : reduce_prev<false>(Pt.res, Pt.gs);
-    if (norm != ASTG_NORM_INF) red = sqrt(red);
-    if (!(red <= DBL_MAX)) {  // a NaN or infinity in b or in the residual: the solve stops (state 4)
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            scal[S_RES] = red;
-            scal[S_ITER] = mode == 0 ? 0.0 : (double)(it + 1);
-            scal[S_DONE] = 4.0;
-        }
-        return true;
-    }
-    if (mode == 0) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            scal[S_BNORM] = red;
-            scal[S_RES] = red;
-            scal[S_TOL] = tolRel * red;
-            scal[S_ITER] = 0;
-            if (red == 0.0) scal[S_DONE] = 1.0;
-        }
-        return red == 0.0;
-    }
-    const bool conv = red <= scal[S_TOL];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        scal[S_RES] = red;
-        scal[S_ITER] = (double)(it + 1);
-        if (conv) scal[S_DONE] = 1.0;
-        else if (it + 1 >= maxIt) scal[S_DONE] = 3.0;
-    }
-    return conv || it + 1 >= maxIt;
-}
-
 // Batched form: a row of a system that has finished takes no part in a sweep.
 __device__ inline bool row_finished(const SweepPlan& S, int i) {
     return S.chunkSys && S.sysState[S.chunkSys[i / BS] * B_COUNT + B_DONE] != 0.0;
@@ -904,6 +867,31 @@ __global__ void k_pad_order(int n, const int* __restrict__ key, const int* __res
     out[gStart[G] + (t - gFirst[G])] = row[t];
 }
 
+__global__ void k_gather_coord(int n, const unsigned long long* coord, const int* perm, unsigned long long* out) {
+    const int i = blockIdx.x * BS + threadIdx.x;
+    if (i < n) out[i] = coord[perm ? perm[i] : i];
+}
+
+int PcgDevice::setCoords(int n, const unsigned long long* coord, const int* ext, std::string& err) {
+    coordExt_[0] = 0;
+    if (!coord) return ASTG_OK;
+    HIPCHK(rowCoord_.alloc((size_t)n * 8));
+    HIPCHK(hipMemcpyAsync(rowCoord_.p, coord, (size_t)n * 8, hipMemcpyHostToDevice, stream_));
+    HIPCHK(hipStreamSynchronize(stream_));
+    for (int a = 0; a < 3; ++a) coordExt_[a] = ext[a];
+    return ASTG_OK;
+}
+
+int PcgDevice::setCoordsDevice(int n, const unsigned long long* coord, const int* perm, const int* ext,
+                               std::string& err) {
+    coordExt_[0] = 0;
+    HIPCHK(rowCoord_.alloc((size_t)n * 8));
+    k_gather_coord<<<blocks(n), BS, 0, stream_>>>(n, coord, perm, rowCoord_.as<unsigned long long>());
+    HIPCHK(hipGetLastError());
+    for (int a = 0; a < 3; ++a) coordExt_[a] = ext[a];
+    return ASTG_OK;
+}
+
 int PcgDevice::setPattern(int n, const int* rowstart, const int* col, std::string& err) {
     if (n <= 0) {
         err = "empty system";
@@ -949,6 +937,8 @@ int PcgDevice::ensureHostPattern(std::string& err) {
 int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const int* dCol, PhaseTimer& tm,
                               std::string& err) {
     f32Valid_ = false;
+    tileCoef64_ = false;
+    tiled_ = false;
     n_ = n;
     nnz_ = nnz;
     if (const char* g = getenv("ASTG_GATE_DIST")) gateDist_ = std::max(1, atoi(g));
@@ -995,7 +985,9 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
     HIPCHK(cnt_.alloc(C_COUNT * 4));
     if (!hscal_) HIPCHK(hipHostMalloc((void**)&hscal_, 32 * 8, hipHostMallocDefault));
     if (!hplan_) HIPCHK(hipHostMalloc((void**)&hplan_, 16 * 8, hipHostMallocDefault));
-    if (dRowstart) {
+    if (dRowstart == rs_.p) {
+        // the pattern is in place (dropTiles)
+    } else if (dRowstart) {
         HIPCHK(hipMemcpyAsync(rs_.p, dRowstart, ((size_t)n + 1) * 4, hipMemcpyDeviceToDevice, stream_));
         HIPCHK(hipMemcpyAsync(col_.p, dCol, (size_t)nnz_ * 4, hipMemcpyDeviceToDevice, stream_));
     } else {
@@ -1139,12 +1131,19 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
         levRange_[2 * L] = lf.gStart[L];
         levRange_[2 * L + 1] = lf.gStart[L] + lf.gRows[L];
     }
-    // sweeps: q levels per group
-    layout(merge_, gateDist_, true, ls);
-    PS_ = ls.P;
-    if (int rc = scatter(ls, merge_, sorder_)) return rc;
-    HIPCHK(upload(sgateF_, ls.gF.data(), ls.gF.size() * 4));
-    HIPCHK(upload(sgateB_, ls.gB.data(), ls.gB.size() * 4));
+    // PCG work vectors: sweep-ordered (PS entries) unless the row order is kept
+    perm_ = !rowOrderForced_;
+    if (const char* g = getenv("ASTG_ROW_ORDER")) perm_ = perm_ && atoi(g) == 0;
+    // sweeps: in tiles where they fit; otherwise q levels per group
+    if (perm_ && !noTile_)
+        if (int rc = tileSetup(tiled_, err)) return rc;
+    if (!tiled_) {
+        layout(merge_, gateDist_, true, ls);
+        PS_ = ls.P;
+        if (int rc = scatter(ls, merge_, sorder_)) return rc;
+        HIPCHK(upload(sgateF_, ls.gF.data(), ls.gF.size() * 4));
+        HIPCHK(upload(sgateB_, ls.gB.data(), ls.gB.size() * 4));
+    }
     if (hostPlan_) {
         // the host construction of both orders and the gates, from the sorted
         // rows, must give the device's entry for entry
@@ -1157,22 +1156,24 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
             err = "device-built factorisation order differs from the host construction";
             return ASTG_ERR_HIP;
         }
-        hostOrder(merge_, gateDist_, n, depth_, sortedLev, sortedRow, spadded, gF, gB);
-        devOrd.resize(PS_);
-        devF.resize(ls.gF.size());
-        devB.resize(ls.gB.size());
-        HIPCHK(hipMemcpyAsync(devOrd.data(), sorder_.p, (size_t)PS_ * 4, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-        if ((int)spadded.size() != PS_ || spadded != devOrd || gF != ls.gF || gB != ls.gB) {
-            err = "device-built sweep order or gates differ from the host construction";
-            return ASTG_ERR_HIP;
+        if (!tiled_) {
+            hostOrder(merge_, gateDist_, n, depth_, sortedLev, sortedRow, spadded, gF, gB);
+            devOrd.resize(PS_);
+            devF.resize(ls.gF.size());
+            devB.resize(ls.gB.size());
+            HIPCHK(hipMemcpyAsync(devOrd.data(), sorder_.p, (size_t)PS_ * 4, hipMemcpyDeviceToHost, stream_));
+            HIPCHK(hipStreamSynchronize(stream_));
+            if ((int)spadded.size() != PS_ || spadded != devOrd || gF != ls.gF || gB != ls.gB) {
+                err = "device-built sweep order or gates differ from the host construction";
+                return ASTG_ERR_HIP;
+            }
         }
     }
     tm.mark("level and sweep orders");
     // symbolic plans: factorisation programs and merged stencils
     const int maxY = kMaxDeps;
     if (!hostPlan_) {
-        const int rc = planDevice(maxY, err);
+        const int rc = planDevice(maxY, !tiled_, err);
         if (rc) return rc;
     } else {
         std::vector<int> lend, ubeg;
@@ -1188,10 +1189,10 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
         HIPCHK(hipStreamSynchronize(stream_));
         std::vector<int> lev(n), pos(n);
         for (int q = 0; q < n; ++q) lev[sortedRow[q]] = sortedLev[q];
-        for (int q = 0; q < PS_; ++q)
+        for (int q = 0; q < PS_ && !tiled_; ++q)
             if (spadded[q] >= 0) pos[spadded[q]] = q;
         DevStencil* dst[2] = {&stF_, &stB_};
-        for (int dir = 0; dir < 2; ++dir) {
+        for (int dir = 0; dir < 2 && !tiled_; ++dir) {
             SweepStencil st;
             planStencil(dir, n, rowstart, lend.data(), ubeg.data(), col, lev.data(), merge_, maxY, spadded.data(),
                         PS_, pos.data(), st);
@@ -1208,9 +1209,6 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
         }
     }
     HIPCHK(live_.alloc((size_t)n));
-    // PCG work vectors: sweep-ordered (PS entries) unless the row order is kept
-    perm_ = !rowOrderForced_;
-    if (const char* g = getenv("ASTG_ROW_ORDER")) perm_ = perm_ && atoi(g) == 0;
     if (perm_) {
         const int rc = permuteSetup(err);
         if (rc) return rc;
@@ -1220,15 +1218,19 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
     HIPCHK(z_.alloc(nv8));
     HIPCHK(s_.alloc(nv8));
     HIPCHK(q_.alloc(nv8));
-    HIPCHK(y_.alloc((size_t)PS_ * 2 * 8));
-    HIPCHK(zp_.alloc((size_t)PS_ * 8));
+    HIPCHK(y_.alloc((size_t)PS_ * (tiled_ ? 1 : 2) * 8));
+    if (!tiled_) HIPCHK(zp_.alloc((size_t)PS_ * 8));
     tm.mark("symbolic plans");
     // persistent grids (all blocks co-resident)
-    const int schunks = PS_ / BS;
-    gF64_ = coopBlocks(k_fwd<double>, cus, schunks);
-    gF32_ = coopBlocks(k_fwd<float>, cus, schunks);
-    gB64_ = coopBlocks(k_bwd_dot<double>, cus, schunks);
-    gB32_ = coopBlocks(k_bwd_dot<float>, cus, schunks);
+    if (tiled_) {
+        gF64_ = gF32_ = gB64_ = gB32_ = tileK_;
+    } else {
+        const int schunks = PS_ / BS;
+        gF64_ = coopBlocks(k_fwd<double>, cus, schunks);
+        gF32_ = coopBlocks(k_fwd<float>, cus, schunks);
+        gB64_ = coopBlocks(k_bwd_dot<double>, cus, schunks);
+        gB32_ = coopBlocks(k_bwd_dot<float>, cus, schunks);
+    }
     gb_ = std::max(std::max(gB64_, gB32_), 1);
     HIPCHK(part_.alloc((size_t)(2 * gs_ + 2 * gb_ + 8) * 8));
     HIPCHK(hipStreamSynchronize(stream_));
@@ -1263,9 +1265,11 @@ int PcgDevice::permuteSetup(std::string& err) {
     HIPCHK(xP_.alloc((size_t)P * 8));
     HIPCHK(permLen_.alloc((size_t)P * 4));
     const int* order = sorder_.as<int>();
-    k_row_pos<<<blocks(P), BS, 0, stream_>>>(P, order, pos_.as<int>());
-    k_rterm_pos<<<blocks(P), BS, 0, stream_>>>(P, stF_.start.as<int>(), stF_.nr.as<int>(), stF_.idx.as<int>(),
-                                               pos_.as<int>());
+    if (!tiled_) {
+        k_row_pos<<<blocks(P), BS, 0, stream_>>>(P, order, pos_.as<int>());
+        k_rterm_pos<<<blocks(P), BS, 0, stream_>>>(P, stF_.start.as<int>(), stF_.nr.as<int>(), stF_.idx.as<int>(),
+                                                   pos_.as<int>());
+    }
     k_perm_len<<<blocks(P), BS, 0, stream_>>>(P, order, rs_.as<int>(), permLen_.as<int>());
     size_t tb = 0;
     HIPCHK(hipcub::DeviceScan::InclusiveSum(nullptr, tb, permLen_.as<int>(), prs_.as<int>() + 1, P, stream_));
@@ -1390,10 +1394,15 @@ int PcgDevice::convert32(std::string& err) {
     const long long nnz = nnz_;
     HIPCHK(val32_.alloc((size_t)nnz * 4));
     HIPCHK(invd32_.alloc((size_t)vlen() * 4));
-    HIPCHK(stF_.coef32.alloc((size_t)stF_.E * 4));
-    HIPCHK(stB_.coef32.alloc((size_t)stB_.E * 4));
     k_d2f<<<blocks(nnz), BS, 0, stream_>>>(sVal64(), val32_.as<float>(), nnz);
     k_d2f<<<blocks(vlen()), BS, 0, stream_>>>(sInvd64(), invd32_.as<float>(), vlen());
+    if (tiled_) {
+        if (int rc = tileCoef<float>(err)) return rc;
+        f32Valid_ = true;
+        return ASTG_OK;
+    }
+    HIPCHK(stF_.coef32.alloc((size_t)stF_.E * 4));
+    HIPCHK(stB_.coef32.alloc((size_t)stB_.E * 4));
     k_d2f<<<blocks(stF_.E), BS, 0, stream_>>>(stF_.coef.as<double>(), stF_.coef32.as<float>(), stF_.E);
     k_d2f<<<blocks(stB_.E), BS, 0, stream_>>>(stB_.coef.as<double>(), stB_.coef32.as<float>(), stB_.E);
     HIPCHK(hipGetLastError());
@@ -1405,7 +1414,8 @@ int PcgDevice::factor(double tau, double ratio, std::string& err) {
     f32Valid_ = false;  // new values and pivots: the FP32 copies are stale
     int rc = launchMic(tau, ratio, err);
     if (rc) return rc;
-    return launchMerge(err);
+    tileCoef64_ = false;  // tile coefficients are gathered by the solve, in its precision
+    return tiled_ ? ASTG_OK : launchMerge(err);
 }
 
 int PcgDevice::syncScalars(std::string& err) {
@@ -1436,6 +1446,35 @@ int PcgDevice::launchBwd(const T* invd, const T* r, T* z, int k, int parityOut, 
     return ASTG_OK;
 }
 
+// A pattern whose tiles fit the LDS in FP32 only, asked for an FP64 solve: the
+// merged sweeps from here on (the values and the factor stay).
+int PcgDevice::dropTiles(std::string& err) {
+    PhaseTimer tm("setPattern (merged sweeps)");
+    noTile_ = true;
+    const int rc = setPatternImpl(n_, nnz_, rs_.as<int>(), col_.as<int>(), tm, err);
+    noTile_ = false;
+    return rc ? rc : launchMerge(err);
+}
+
+// The values that the first sweep of a solve waits for.
+template <typename T>
+void PcgDevice::armSweeps() {
+    if (!tiled_) {
+        k_fill_sent<T><<<blocks(2 * PS_), BS, 0, stream_>>>(y_.as<T>(), 2 * PS_);
+        return;
+    }
+    for (int d = 0; d < 2; ++d)
+        if (const int h = 2 * tile_[d].halo) k_fill_sent<T><<<blocks(h), BS, 0, stream_>>>(tile_[d].inbox.as<T>(), h);
+}
+
+template <typename T>
+int PcgDevice::precondition(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm,
+                            double tolRel, std::string& err) {
+    if (tiled_) return launchTile<T>(invd, r, z, k, mode, it, maxIt, norm, tolRel, 3, err);
+    if (int rc = launchFwd<T>(invd, r, k, mode, it, maxIt, norm, tolRel, err)) return rc;
+    return launchBwd<T>(invd, r, z, k, k & 1, err);
+}
+
 template <typename T>
 int PcgDevice::pcgInner(const T* A, const T* invd, const T* b, double* x, double tolRel, int maxIt, int norm,
                         int& iters, double& resOut, bool& conv, std::string& err, const double* b64,
@@ -1453,9 +1492,8 @@ int PcgDevice::pcgInner(const T* A, const T* invd, const T* b, double* x, double
     int rc;
     k_zero64<<<1, BS, 0, stream_>>>(32, scal);
     k_init<T, double><<<gs, BS, 0, stream_>>>(n, b, x, r, Pt, norm);
-    k_fill_sent<T><<<blocks(2 * PS_), BS, 0, stream_>>>(y_.as<T>(), 2 * PS_);
-    if ((rc = launchFwd<T>(invd, r, 0, 0, 0, maxIt, norm, tolRel, err))) return rc;
-    if ((rc = launchBwd<T>(invd, r, z, 0, 0, err))) return rc;
+    armSweeps<T>();
+    if ((rc = precondition<T>(invd, r, z, 0, 0, 0, maxIt, norm, tolRel, err))) return rc;
     if (forceSpinError_ && !coop_) {  // test hook: as if a sweep had hit its spin limit
         forceSpinError_ = false;
         k_set_err<<<1, 64, 0, stream_>>>(cnt_.as<int>(), E_FWD);
@@ -1464,9 +1502,9 @@ int PcgDevice::pcgInner(const T* A, const T* invd, const T* b, double* x, double
     // failure is caught here, before any iteration is spent on it
     rc = checkErrors("PCG", err);
     if (rc) return rc;
-    // z as the PCG reads it: the backward sweep's published copy in sweep
-    // order (valid until the next forward sweep re-arms it)
-    const T* zv = perm_ ? zp_.as<T>() : z;
+    // z as the PCG reads it: with merged sweeps in sweep order the backward
+    // sweep's published copy (valid until the next forward sweep re-arms it)
+    const T* zv = perm_ && !tiled_ ? zp_.as<T>() : z;
     k_xpby<T><<<gs, BS, 0, stream_>>>(n, zv, s, Pt, scal, 0, 0);
     HIPCHK(hipGetLastError());
     int it = 0;
@@ -1478,8 +1516,7 @@ int PcgDevice::pcgInner(const T* A, const T* invd, const T* b, double* x, double
             if (sizeof(T) == 4 && replaceEvery > 0 && (it + 1) % replaceEvery == 0)
                 k_replace_res<<<gs, BS, 0, stream_>>>(n, rs, col, sVal64(), x, b64,
                                                       reinterpret_cast<float*>(r), Pt, scal, norm);
-            if ((rc = launchFwd<T>(invd, r, it + 1, 1, it, maxIt, norm, tolRel, err))) return rc;
-            if ((rc = launchBwd<T>(invd, r, z, it + 1, (it + 1) & 1, err))) return rc;
+            if ((rc = precondition<T>(invd, r, z, it + 1, 1, it, maxIt, norm, tolRel, err))) return rc;
             k_xpby<T><<<gs, BS, 0, stream_>>>(n, zv, s, Pt, scal, 1, it);
         }
         HIPCHK(hipGetLastError());
@@ -1514,6 +1551,14 @@ int PcgDevice::solve(const astg_pcg_params& prm, astg_pcg_result& res, std::stri
 }
 
 int PcgDevice::solveOnce(const astg_pcg_params& prm, astg_pcg_result& res, std::string& err) {
+    if (tiled_ && prm.precision == ASTG_PREC_FP64) {
+        if (!tilesFit(tileSlots_, 8)) {
+            if (int rc = dropTiles(err)) return rc;
+        } else if (!tileCoef64_) {
+            if (int rc = tileCoef<double>(err)) return rc;
+            tileCoef64_ = true;
+        }
+    }
     const int n = vlen(), gs = gs_;
     res.n = n_;
     res.nnz = nnz_;
@@ -1635,7 +1680,7 @@ int PcgDevice::downloadFactor(std::vector<double>& invdiag, std::vector<unsigned
 }
 
 int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, std::string& err) {
-    const int n = n_, gs = gs_, nv = vlen();
+    const int n = n_, nv = vlen();
     const long long nnz = nnz_, nl = nnzL();
     // the solve's own layout: sweep-ordered vectors and CSR unless the row order is kept
     if (int rc = prepareSolve(err)) return rc;
@@ -1647,22 +1692,57 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
         int rc = convert32(err);
         if (rc) return rc;
     }
+    if (tiled_ && (which == ASTG_K_FWD64 || which == ASTG_K_BWD64)) {
+        if (!tilesFit(tileSlots_, 8)) {
+            err = "the FP64 sweeps of this ordering need a FP64 solve first";
+            return ASTG_ERR_STATE;
+        }
+        if (!tileCoef64_) {
+            if (int rc = tileCoef<double>(err)) return rc;
+            tileCoef64_ = true;
+        }
+    }
+    // one direction of a sweep
+    auto sweep64 = [&](int dir) -> int {
+        const double* iv = sInvd64();
+        if (tiled_)
+            return launchTile<double>(iv, r_.as<double>(), z_.as<double>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30,
+                                      1 << dir, err);
+        return dir == 0 ? launchFwd<double>(iv, r_.as<double>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30, err)
+                        : launchBwd<double>(iv, r_.as<double>(), z_.as<double>(), 0, 0, err);
+    };
+    auto sweep32 = [&](int dir) -> int {
+        const float* iv = invd32_.as<float>();
+        if (tiled_)
+            return launchTile<float>(iv, r_.as<float>(), z_.as<float>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30,
+                                     1 << dir, err);
+        return dir == 0 ? launchFwd<float>(iv, r_.as<float>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30, err)
+                        : launchBwd<float>(iv, r_.as<float>(), z_.as<float>(), 0, 0, err);
+    };
     const double w = f32 ? 4.0 : 8.0;
     switch (which) {
         case ASTG_K_SPMV64: case ASTG_K_SPMV32:
             // values + columns, rowstart, s gathered once, s read for the dot, q written
             bytes = (w + 4) * nnz + 4.0 * (n + 1) + 3 * w * n;
             break;
-        case ASTG_K_FWD64: case ASTG_K_FWD32:
+        case ASTG_K_FWD64: case ASTG_K_FWD32: case ASTG_K_BWD64: case ASTG_K_BWD32:
+            if (tiled_) {
+                // coefficients + slots of the stored entries; per position: r or y, pivot, y or z
+                // written, gate, flag (backward also r for the dot); per halo entry: source, value
+                const bool bw = which == ASTG_K_BWD64 || which == ASTG_K_BWD32;
+                bytes = (w + 2) * tile_[bw ? 1 : 0].E + ((bw ? 4.0 : 3.0) * w + 3) * PS_;
+                break;
+            }
+            if (which == ASTG_K_BWD64 || which == ASTG_K_BWD32) {
+                // stencil coefficients + indices; per row: order, start, r-term count, y, next y
+                // armed, pivot, r, z published (and, in row order, written to the PCG vector),
+                // z gathered once
+                bytes = (w + 4) * stB_.E + ((perm_ ? 6.0 : 7.0) * w + 12) * n;
+                break;
+            }
             // stencil coefficients + indices; per row: order, start, r-term count, r, pivot,
             // y written, y gathered once, backward vector armed
             bytes = (w + 4) * stF_.E + (5.0 * w + 12) * n;
-            break;
-        case ASTG_K_BWD64: case ASTG_K_BWD32:
-            // stencil coefficients + indices; per row: order, start, r-term count, y, next y
-            // armed, pivot, r, z published (and, in row order, written to the PCG vector),
-            // z gathered once
-            bytes = (w + 4) * stB_.E + ((perm_ ? 6.0 : 7.0) * w + 12) * n;
             break;
         case ASTG_K_MIC:
             // A values + pattern read, factor written twice (both triangles), invd
@@ -1687,19 +1767,19 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
         // re-arm the device state so no kernel early-exits
         k_zero64<<<1, BS, 0, stream_>>>(32, scal);
         const Parts P64 = parts(bwdGrid<double>()), P32 = parts(bwdGrid<float>());
-        if (which == ASTG_K_FWD64 || which == ASTG_K_BWD64) {
-            k_fill_sent<double><<<blocks(2 * PS_), BS, 0, stream_>>>(y_.as<double>(), 2 * PS_);
-            k_fill_sent<double><<<blocks(PS_), BS, 0, stream_>>>(zp_.as<double>(), PS_);
-        } else if (which == ASTG_K_FWD32 || which == ASTG_K_BWD32) {
-            k_fill_sent<float><<<blocks(2 * PS_), BS, 0, stream_>>>(y_.as<float>(), 2 * PS_);
-            k_fill_sent<float><<<blocks(PS_), BS, 0, stream_>>>(zp_.as<float>(), PS_);
+        if (sweep && f32) {
+            armSweeps<float>();
+            if (!tiled_) k_fill_sent<float><<<blocks(PS_), BS, 0, stream_>>>(zp_.as<float>(), PS_);
+        } else if (sweep) {
+            armSweeps<double>();
+            if (!tiled_) k_fill_sent<double><<<blocks(PS_), BS, 0, stream_>>>(zp_.as<double>(), PS_);
         }
         // the forward sweep starts in mode 0, which needs nonzero ||b|| partials
         if (sweep) k_fill64<<<blocks(gs_), BS, 0, stream_>>>(gs_, P64.res, 1.0);
         if (which == ASTG_K_BWD64)
-            rc = launchFwd<double>(sInvd64(), r_.as<double>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30, err);
+            rc = sweep64(0);
         else if (which == ASTG_K_BWD32)
-            rc = launchFwd<float>(invd32_.as<float>(), r_.as<float>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30, err);
+            rc = sweep32(0);
         if (rc) break;
         HIPCHK(hipEventRecord(e0, stream_));
         switch (which) {
@@ -1712,17 +1792,16 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
                                                           q_.as<float>(), P32, scal);
                 break;
             case ASTG_K_FWD64:
-                rc = launchFwd<double>(sInvd64(), r_.as<double>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30, err);
+                rc = sweep64(0);
                 break;
             case ASTG_K_FWD32:
-                rc = launchFwd<float>(invd32_.as<float>(), r_.as<float>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30,
-                                      err);
+                rc = sweep32(0);
                 break;
             case ASTG_K_BWD64:
-                rc = launchBwd<double>(sInvd64(), r_.as<double>(), z_.as<double>(), 0, 0, err);
+                rc = sweep64(1);
                 break;
             case ASTG_K_BWD32:
-                rc = launchBwd<float>(invd32_.as<float>(), r_.as<float>(), z_.as<float>(), 0, 0, err);
+                rc = sweep32(1);
                 break;
             case ASTG_K_MIC:
                 rc = launchMic(0.97, 0.25, err);

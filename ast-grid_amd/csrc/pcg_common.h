@@ -4,9 +4,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
 #include <string>
 
 #include "device_common.h"
+#include "pcg.h"
 
 #define HIPCHK(expr)                                                                 \
     do {                                                                             \
@@ -25,25 +27,63 @@ constexpr int kLpr = 8;  // lanes per row in the SpMV kernels
 // ---------------------------------------------------------------------------
 // deterministic block reductions
 // ---------------------------------------------------------------------------
-template <bool MAX>
+template <bool MAX, int NT = BS>
 __device__ inline double block_reduce(double v) {
-    __shared__ double sm[BS / 64];
+    __shared__ double sm[NT / 64];
     v = MAX ? wave_max(v) : wave_sum(v);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __syncthreads();  // sm may still be read by a previous call
     if (lane == 0) sm[wid] = v;
     __syncthreads();
     double t = sm[0];
-    for (int w = 1; w < BS / 64; ++w) t = MAX ? nan_max(t, sm[w]) : t + sm[w];
+    for (int w = 1; w < NT / 64; ++w) t = MAX ? nan_max(t, sm[w]) : t + sm[w];
     return t;
 }
 // Sum (or max) of np partials written by the previous kernel, same order in
 // every block.
-template <bool MAX>
+template <bool MAX, int NT = BS>
 __device__ inline double reduce_prev(const double* part, int np) {
     double acc = 0.0;
-    for (int s = threadIdx.x; s < np; s += BS) acc = MAX ? nan_max(acc, part[s]) : acc + part[s];
-    return block_reduce<MAX>(acc);
+    for (int s = threadIdx.x; s < np; s += NT) acc = MAX ? nan_max(acc, part[s]) : acc + part[s];
+    return block_reduce<MAX, NT>(acc);
+}
+
+// Forward sweep y = L^-1 r. mode 0 (start of the solve): ||b|| from the
+// partials, tolerance, zero-rhs exit. mode 1 (iteration `it`): the reference's
+// convergence test on the updated residual, before preconditioning. mode 2:
+// no test here (the batched solve tests each system in its own kernel).
+// Returns true when the solve stops here (every block takes the same decision).
+template <int NT = BS>
+__device__ inline bool fwd_prologue(const Parts& Pt, double* scal, int mode, int it, int maxIt, int norm,
+                                    double tolRel) {
+    double red = norm == ASTG_NORM_INF ? reduce_prev<true, NT>(Pt.res, Pt.gs) : reduce_prev<false, NT>(Pt.res, Pt.gs);
+    if (norm != ASTG_NORM_INF) red = sqrt(red);
+    if (!(red <= DBL_MAX)) {  // a NaN or infinity in b or in the residual: the solve stops (state 4)
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            scal[S_RES] = red;
+            scal[S_ITER] = mode == 0 ? 0.0 : (double)(it + 1);
+            scal[S_DONE] = 4.0;
+        }
+        return true;
+    }
+    if (mode == 0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            scal[S_BNORM] = red;
+            scal[S_RES] = red;
+            scal[S_TOL] = tolRel * red;
+            scal[S_ITER] = 0;
+            if (red == 0.0) scal[S_DONE] = 1.0;
+        }
+        return red == 0.0;
+    }
+    const bool conv = red <= scal[S_TOL];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        scal[S_RES] = red;
+        scal[S_ITER] = (double)(it + 1);
+        if (conv) scal[S_DONE] = 1.0;
+        else if (it + 1 >= maxIt) scal[S_DONE] = 3.0;
+    }
+    return conv || it + 1 >= maxIt;
 }
 
 // (A s)_i with LPR lanes per row (rows are short: 8 entries on average), so

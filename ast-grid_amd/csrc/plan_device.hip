@@ -25,7 +25,7 @@ inline int grid(long n, int bs) { return (int)((n + bs - 1) / bs); }
 
 using namespace plan;
 
-int PcgDevice::planDevice(int maxY, std::string& err) {
+int PcgDevice::planDevice(int maxY, bool stencils, std::string& err) {
     if (maxY > kMaxDeps) {
         err = "sweep stencil: maxY above the dependency limit";
         return ASTG_ERR_ARG;
@@ -47,6 +47,7 @@ int PcgDevice::planDevice(int maxY, std::string& err) {
     int* cI[2] = {planCnt_.as<int>(), planCnt_.as<int>() + 2 * (size_t)P};
     int* cU[2] = {planCnt_.as<int>() + (size_t)P, planCnt_.as<int>() + 3 * (size_t)P};
     for (DevStencil* D : dst) {
+        if (!stencils) break;
         HIPCHK(D->start.alloc(((size_t)P + 1) * 4));
         HIPCHK(D->ustart.alloc(((size_t)P + 1) * 4));
         HIPCHK(D->nr.alloc((size_t)P * 4));
@@ -54,7 +55,8 @@ int PcgDevice::planDevice(int maxY, std::string& err) {
     long long* mstart = micStart_.as<long long>();
     size_t b64 = 0, b32 = 0;
     HIPCHK(hipcub::DeviceScan::InclusiveSum(nullptr, b64, planLen_.as<long long>(), mstart + 1, (int)nnz, stream_));
-    HIPCHK(hipcub::DeviceScan::InclusiveSum(nullptr, b32, cI[0], dst[0]->start.as<int>() + 1, P, stream_));
+    if (stencils)
+        HIPCHK(hipcub::DeviceScan::InclusiveSum(nullptr, b32, cI[0], dst[0]->start.as<int>() + 1, P, stream_));
     size_t tb = std::max(b64, b32);
     HIPCHK(planTmp_.alloc(tb));
     // count passes and prefix sums
@@ -63,8 +65,9 @@ int PcgDevice::planDevice(int maxY, std::string& err) {
     HIPCHK(hipcub::DeviceScan::InclusiveSum(planTmp_.p, tb, planLen_.as<long long>(), mstart + 1, (int)nnz,
                                             stream_));
     k_set_i64<<<1, 64, 0, stream_>>>(mstart, 0);
-    k_sweep_pos<<<grid(P, 256), 256, 0, stream_>>>(P, order, planPos_.as<int>());
-    for (int dir = 0; dir < 2; ++dir) {
+    const int ndir = stencils ? 2 : 0;
+    if (stencils) k_sweep_pos<<<grid(P, 256), 256, 0, stream_>>>(P, order, planPos_.as<int>());
+    for (int dir = 0; dir < ndir; ++dir) {
         DevStencil& D = *dst[dir];
         auto kc = dir == 0 ? k_plan_stencil<0, false> : k_plan_stencil<1, false>;
         kc<<<grid(P, 64), 64, 0, stream_>>>(P, rs, lend, ubeg, col, lev, merge_, maxY, order, planPos_.as<int>(),
@@ -79,7 +82,7 @@ int PcgDevice::planDevice(int maxY, std::string& err) {
     // sizes: program length, entries and slots per direction, error flag
     int* hi = reinterpret_cast<int*>(hplan_ + 1);
     HIPCHK(hipMemcpyAsync(hplan_, mstart + nnz, 8, hipMemcpyDeviceToHost, stream_));
-    for (int dir = 0; dir < 2; ++dir) {
+    for (int dir = 0; dir < ndir; ++dir) {
         HIPCHK(hipMemcpyAsync(hi + 2 * dir, dst[dir]->start.as<int>() + P, 4, hipMemcpyDeviceToHost, stream_));
         HIPCHK(hipMemcpyAsync(hi + 2 * dir + 1, dst[dir]->ustart.as<int>() + P, 4, hipMemcpyDeviceToHost, stream_));
     }
@@ -92,7 +95,7 @@ int PcgDevice::planDevice(int maxY, std::string& err) {
     // fill passes
     HIPCHK(micProg_.alloc((size_t)hplan_[0] * 4));
     k_plan_mic<true><<<grid(n, 256), 256, 0, stream_>>>(n, rs, lend, ubeg, col, nullptr, mstart, micProg_.as<int>());
-    for (int dir = 0; dir < 2; ++dir) {
+    for (int dir = 0; dir < ndir; ++dir) {
         DevStencil& D = *dst[dir];
         D.E = hi[2 * dir];
         HIPCHK(D.idx.alloc((size_t)D.E * 4));

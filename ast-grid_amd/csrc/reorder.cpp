@@ -56,6 +56,25 @@ void blockKeys(const Octree& o, const Numbering& num, int blockCells, std::vecto
     });
 }
 
+void rowCoords(const Octree& o, const Numbering& num, std::vector<unsigned long long>& coord, int* ext) {
+    for (int a = 0; a < 3; ++a) ext[a] = 2 * o.R + 1;
+    coord.assign(num.n, 0ull);
+    for (int l = 0; l < o.L; ++l) {
+        const Level& Lv = o.lv[l];
+        const unsigned long long s = 2ull << l, h = s >> 1;
+        parallelFor(Lv.nnode, [&](long i0, long i1) {
+            for (long i = i0; i < i1; ++i) {
+                const int a = num.oct[l][i], t = num.tilt[l][i];
+                const unsigned long long x = Lv.x[i] * s, y = Lv.y[i] * s, z = Lv.z[i] * s;
+                // nodes sharing a row (a vertex on several levels) are at one position
+                if (a >= 0)
+                    __atomic_store_n(&coord[a], (z + h) << 36 | (y + h) << 18 | (x + h), __ATOMIC_RELAXED);
+                if (t >= 0) __atomic_store_n(&coord[t], z << 36 | y << 18 | x, __ATOMIC_RELAXED);
+            }
+        });
+    }
+}
+
 void buildBlockOrder(const Octree& o, const Numbering& num, const std::vector<int>& rowstart,
                      const std::vector<int>& col, int blockCells, BlockOrder& out) {
     const int n = num.n;

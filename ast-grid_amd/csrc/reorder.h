@@ -39,6 +39,10 @@ struct BlockOrder {
 void buildBlockOrder(const Octree& o, const Numbering& num, const std::vector<int>& rowstart,
                      const std::vector<int>& col, int blockCells, BlockOrder& out);
 
+// Position of every row on the doubled finest grid (cell centres odd), packed
+// z << 36 | y << 18 | x, and the extents; a row without a node is at the origin.
+void rowCoords(const Octree& o, const Numbering& num, std::vector<unsigned long long>& coord, int* ext);
+
 // The sort key of every row of the reference numbering: colour * cubes + cube
 // of the row's position (the first node, in level and node order, that holds
 // the row), 8 * cubes for a row without one. Host worker pool. buildBlockOrder

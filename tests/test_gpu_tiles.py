@@ -1,0 +1,118 @@
+"""Tiled sweeps against the CPU oracle's PCG at the sizes where the tiling can
+go wrong: fewer rows than a wavefront, chunks of exactly 64 rows and one more
+or less, one tile and many, tiles of a single chunk, rows without entries on
+one side, two- and three-dimensional patterns, both precisions. The merged
+sweeps (ASTG_TILES=0) are the reference for the octree and uniform forms.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def box(shape, rng, diagonals=False):
+    """SPD matrix of a box (x fastest): 7-point, or 27-point with diagonals."""
+    nz, ny, nx = shape
+    idx = np.arange(nz * ny * nx).reshape(shape)
+    off = [(0, 0, 1), (0, 1, 0), (1, 0, 0)]
+    if diagonals:
+        off += [(0, 1, 1), (0, 1, -1), (1, 0, 1), (1, 0, -1), (1, 1, 0), (1, -1, 0)]
+    n = idx.size
+    rows, cols, vals = [np.arange(n)], [np.arange(n)], [np.zeros(n)]
+    diag = np.full(n, 0.05)
+    for d in off:
+        a = idx[tuple(slice(max(0, -v), s - max(0, v)) for v, s in zip(d, shape))].ravel()
+        b = idx[tuple(slice(max(0, v), s - max(0, -v)) for v, s in zip(d, shape))].ravel()
+        w = rng.uniform(0.2, 1.0, a.size)
+        rows += [a, b]
+        cols += [b, a]
+        vals += [-w, -w]
+        np.add.at(diag, a, w)
+        np.add.at(diag, b, w)
+    r, c, v = np.concatenate(rows), np.concatenate(cols), np.concatenate(vals)
+    v[:n] = diag
+    o = np.lexsort((c, r))
+    rs = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]).astype(np.int32)
+    return rs, c[o].astype(np.int32), v[o]
+
+
+CASES = [
+    ((1, 1, 1), 1), ((1, 1, 63), 1), ((1, 1, 64), 1), ((1, 1, 65), 2), ((1, 5, 13), 3), ((3, 5, 7), 4),
+    ((4, 4, 4), 64), ((8, 8, 8), 1), ((8, 8, 8), 8), ((9, 11, 13), 5), ((16, 16, 16), 31), ((5, 40, 41), 64),
+    ((21, 22, 23), 7), ((1, 120, 121), 16), ((40, 41, 42), 256),
+]
+
+
+@pytest.mark.parametrize("diagonals", [False, True], ids=["7pt", "19pt"])
+@pytest.mark.parametrize("shape,tiles", CASES)
+def test_csr_matches_oracle(shape, tiles, diagonals, monkeypatch):
+    import astg
+    from oracle import oracle as orc
+    rng = np.random.default_rng(shape[0] * 7 + tiles)
+    rs, col, val = box(shape, rng, diagonals)
+    n = len(rs) - 1
+    b = rng.standard_normal(n)
+    tol = 1e-12
+    monkeypatch.setenv("ASTG_TILES", str(tiles))
+    c = astg.Context(0)
+    x, r = c.pcg_solve_csr(rs, col, val, b, astg.default_params(tol=tol, max_iterations=3000))
+    xm, rm = c.pcg_solve_csr(rs, col, val, b, astg.default_params(tol=tol, max_iterations=3000,
+                                                                  precision=astg.PREC_MIXED))
+    c.close()
+    want, _, iters, ok = orc.pcg(rs, col, val, b, tol=tol)
+    assert ok
+    # The diagonal exceeds the row's off-diagonal sum by 0.05, so the smallest
+    # eigenvalue is at least 0.05, and ||x - x'||inf <= ||r||inf / 0.05 for a
+    # diagonally dominant matrix: 2 tol ||b|| / 0.05 for two solves.
+    bound = 2 * tol * np.abs(b).max() / 0.05
+    assert r.converged == 1 and abs(r.iterations - iters) <= 1
+    assert np.abs(x - want).max() <= bound
+    assert rm.converged == 1 and np.abs(xm - want).max() <= bound
+
+
+@pytest.mark.parametrize("precision,ordering", [("fp64", 1), ("fp64", 2), ("mixed", 1), ("mixed", 2)])
+@pytest.mark.parametrize("tiles", [1, 5, 27, 200])
+def test_octree_matches_merged_sweeps(tiles, precision, ordering, monkeypatch):
+    """The same preconditioner through tiles and through merged sweeps: the
+    iterates agree up to rounding, so the iteration counts do."""
+    import astg
+    from astg import scenes
+    out = []
+    for t in (0, tiles):
+        monkeypatch.setenv("ASTG_TILES", str(t))
+        ctx, info = scenes.smoke_64(device=0)
+        scenes.fill_velocity(ctx, info["levels"], 3)
+        prm = astg.default_params(tol=1e-10, max_iterations=3000, ordering=ordering,
+                                  precision=astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64)
+        res = ctx.project(info["dt"], info["rho"], prm)
+        out.append((res.iterations, ctx.system(res.n, res.nnz)[4]))
+        ctx.close()
+    (i0, p0), (i1, p1) = out
+    assert abs(i0 - i1) <= (1 if precision == "fp64" else 4)
+    # both residuals are 1e-10 of b; the systems' condition is below 1e4 here
+    assert np.linalg.norm(p1 - p0) <= 2e-6 * np.linalg.norm(p0)
+
+
+@pytest.mark.parametrize("res", [(34, 21), (19, 18, 17)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_uniform_matches_merged_sweeps(res, precision, monkeypatch):
+    import astg
+    from astg import uniform
+    rng = np.random.default_rng(5)
+    d = len(res)
+    open_ = (rng.random(int(np.prod([r + 1 for r in res]))) < 0.3).astype(np.uint8)
+    mac = [rng.standard_normal(int(np.prod([r + (i == a) for i, r in enumerate(res)]))) for a in range(d)]
+    tilt = rng.standard_normal((open_.size, 4 if d == 2 else 8))
+    out = []
+    for t in (0, 1, 7):
+        monkeypatch.setenv("ASTG_TILES", str(t))
+        s = uniform.ASTSolver(d, res, 1.0 / res[0])
+        s.set_layout(open_)
+        s.set_velocity(mac, tilt)
+        prm = uniform.default_params(precision=astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64,
+                                     tol=1e-9)
+        r = s.project(0.025, 2.0, prm)
+        out.append((r.iterations, np.concatenate([u.ravel() for u in s.velocity()[0]])))
+    for it, u in out[1:]:
+        assert abs(it - out[0][0]) <= (1 if precision == "fp64" else 4)
+        assert np.abs(u - out[0][1]).max() <= 1e-7 * np.abs(u).max()
