@@ -1574,8 +1574,16 @@ static __device__ __align__(256) double scratch[(size_t)kNoAllocPoints * 6];
 // sampled position. The transpose of a sampler at a point is applied by
 // probing: run k of the sampler returns 1 for its k-th load and 0 for the
 // others, so its output is that load's weight, which is scattered (atomic
-// add) into the adjoint of the loaded entry. The derivative with respect to
+// add) into the adjoint of the loaded entry. The runs of one degree of freedom
+// are shared by kAdjLanes neighbouring lanes: lane `sub` takes runs sub, sub +
+// kAdjLanes, .... (A degree of freedom makes 100 to 250 runs of a chain of
+// dependent gathers; one lane each left most of the chip idle and the lanes of
+// a wavefront on 64 different paths. A rollout of 3 steps and its gradient, ms
+// at 1 / 4 / 8 / 16 / 32 lanes: 32^3 102 / 47 / 39 / 36 / 34, 64^3 123 / 64 /
+// 56 / 52 / 51; 2 steps at 128^3 89 / 60 / 57 / 56 / 57.) The derivative with respect to
 // the position comes from the same sampler evaluated on D3 positions.
+constexpr int kAdjLanes = 16;
+
 struct ProbeLd {
     int target;
     int cnt = 0;
@@ -1613,16 +1621,17 @@ __device__ inline D3 seed(double v, int k) {
 }
 
 // Scatters sum_c ubar[c] * d out[c] / d field into the adjoints, out = U(p).
-__device__ __noinline__ void velSampleTranspose(const Topo& T, const Vel& V, const AdjMap& A, const double* p, const double* ubar) {
+__device__ __noinline__ void velSampleTranspose(const Topo& T, const Vel& V, const AdjMap& A, const double* p,
+                                                const double* ubar, int sub) {
     if (ubar[0] == 0.0 && ubar[1] == 0.0 && ubar[2] == 0.0) return;
     double o[3];
-    ProbeLd c0(-1);
-    velSampleT(T, V, c0, p[0], p[1], p[2], o);
-    for (int k = 0; k < c0.cnt; ++k) {
+    // every run counts the sampler's loads; run k past them changes nothing
+    for (int k = sub, loads = 0; k == sub || k < loads; k += kAdjLanes) {
         ProbeLd pk(k);
         velSampleT(T, V, pk, p[0], p[1], p[2], o);
+        loads = pk.cnt;
         const double w = ubar[0] * o[0] + ubar[1] * o[1] + ubar[2] * o[2];
-        if (w != 0.0 && isfinite(w)) {
+        if (pk.tb && w != 0.0 && isfinite(w)) {
             double* a = A.of(pk.tb);
             if (a) atomicAdd(a + pk.ti, w);
         }
@@ -1645,13 +1654,13 @@ __device__ __noinline__ void velSampleGradT(const Topo& T, const Vel& V, const d
 // given qbar = d loss / d q, scatters the velocity-field adjoints of both
 // velocity samples (at p and at the midpoint).
 __device__ __noinline__ void backTraceAdjoint(const Topo& T, const Vel& V, const AdjMap& A, const double* p, double dt,
-                                 const double* mid, const double* qbar) {
+                                 const double* mid, const double* qbar, int sub) {
     double v2bar[3], mbar[3], v1bar[3];
     for (int c = 0; c < 3; ++c) v2bar[c] = -dt * qbar[c];
-    velSampleTranspose(T, V, A, mid, v2bar);
+    velSampleTranspose(T, V, A, mid, v2bar, sub);
     velSampleGradT(T, V, mid, v2bar, mbar);
     for (int c = 0; c < 3; ++c) v1bar[c] = -dt * 0.5 * mbar[c];
-    velSampleTranspose(T, V, A, p, v1bar);
+    velSampleTranspose(T, V, A, p, v1bar, sub);
 }
 
 // The forward back-trace with its midpoint (no collider on this path)
@@ -1666,7 +1675,8 @@ __device__ __noinline__ void traceFwd(const Topo& T, const Vel& V, const double*
 __global__ void k_adj_adv_scalar(Topo T, const uint8_t* level, Vel V, AdjMap A, const int* list, int n, int kind,
                                  double dt, const double* d0c, const double* d0v, const double* rbarAdv, double* rbarC,
                                  double* rbarV, const uint8_t* skipHalf) {
-    const int t = blockIdx.x * BS + threadIdx.x;
+    const long tt = (long)blockIdx.x * BS + threadIdx.x;
+    const int t = (int)(tt / kAdjLanes), sub = (int)(tt % kAdjLanes);
     if (t >= n) return;
     const int g = list[t];
     if (skipHalf && skipHalf[g]) return;
@@ -1686,12 +1696,11 @@ __global__ void k_adj_adv_scalar(Topo T, const uint8_t* level, Vel V, AdjMap A, 
     traceFwd(T, V, p, dt, mid, q);
     // S^T at q into the density adjoints
     {
-        ProbeLd c0(-1);
-        scalarSampleT(T, c0, d0c, d0v, q[0], q[1], q[2]);
-        for (int k = 0; k < c0.cnt; ++k) {
+        for (int k = sub, loads = 0; k == sub || k < loads; k += kAdjLanes) {
             ProbeLd pk(k);
             const double w = ab * scalarSampleT(T, pk, d0c, d0v, q[0], q[1], q[2]);
-            if (w != 0.0 && isfinite(w)) atomicAdd((pk.tb == d0c ? rbarC : rbarV) + pk.ti, w);
+            loads = pk.cnt;
+            if (pk.tb && w != 0.0 && isfinite(w)) atomicAdd((pk.tb == d0c ? rbarC : rbarV) + pk.ti, w);
         }
     }
     // position gradient at q, then the back-trace
@@ -1699,20 +1708,20 @@ __global__ void k_adj_adv_scalar(Topo T, const uint8_t* level, Vel V, AdjMap A, 
     const D3 sv = scalarSampleT(T, ld, d0c, d0v, seed(q[0], 0), seed(q[1], 1), seed(q[2], 2));
     double qbar[3];
     for (int k = 0; k < 3; ++k) qbar[k] = isfinite(sv.d[k]) ? ab * sv.d[k] : 0.0;
-    backTraceAdjoint(T, V, A, p, dt, mid, qbar);
+    backTraceAdjoint(T, V, A, p, dt, mid, qbar, sub);
 }
 
-// Adjoint of the velocity advection: kind 0 MAC face (axis = sub), 1 tilt
-// slot (slot = sub), 2 half-tilt slot (slot = sub, face slot at i == 4).
+// Adjoint of the velocity advection: kind 0 MAC face (axis = slot), 1 tilt
+// slot, 2 half-tilt slot (face slot at slot == 4).
 __device__ void advVelDof(const Topo& T, const double* teDst, const uint8_t* level, const Vel& V, const AdjMap& A,
-                          int g, int kind, int sub, double dt, double ab) {
+                          int g, int kind, int slot, double dt, double ab, int sub) {
     const int l = level[g];
     const double h = c_hl[l];
     int x, y, z;
     nodeXYZ(T, g, x, y, z);
     double p[3], d[3] = {0, 0, 0};
     if (kind == 0) {
-        const int a = sub;
+        const int a = slot;
         p[0] = x * h + (a == 0 ? 0.0 : 0.5) * h;
         p[1] = y * h + (a == 1 ? 0.0 : 0.5) * h;
         p[2] = z * h + (a == 2 ? 0.0 : 0.5) * h;
@@ -1720,8 +1729,8 @@ __device__ void advVelDof(const Topo& T, const double* teDst, const uint8_t* lev
     } else {
         const double c[3] = {x * h, y * h, z * h};
         const int dir = T.thd[g];
-        const int k = kind == 1 ? sub : c_halfSlot[dir][sub];
-        if (kind == 2 && sub == 4) {
+        const int k = kind == 1 ? slot : c_halfSlot[dir][slot];
+        if (kind == 2 && slot == 4) {
             p[0] = c[0], p[1] = c[1], p[2] = c[2];
             const int ax = (k == 0 || k == 1) ? 0 : (k == 2 || k == 4) ? 1 : 2;
             d[ax] = 1.0;
@@ -1733,40 +1742,40 @@ __device__ void advVelDof(const Topo& T, const double* teDst, const uint8_t* lev
     double mid[3], q[3];
     traceFwd(T, V, p, dt, mid, q);
     double ubar[3] = {ab * d[0], ab * d[1], ab * d[2]}, qbar[3];
-    velSampleTranspose(T, V, A, q, ubar);
+    velSampleTranspose(T, V, A, q, ubar, sub);
     velSampleGradT(T, V, q, ubar, qbar);
-    backTraceAdjoint(T, V, A, p, dt, mid, qbar);
+    backTraceAdjoint(T, V, A, p, dt, mid, qbar, sub);
 }
 
 __global__ void k_adj_adv_mac(Topo T, const double* teDst, const uint8_t* level, Vel V, AdjMap A, const int* leafList,
                               int n, double dt, const double* ubarMac) {
-    const int t = blockIdx.x * BS + threadIdx.x;
-    if (t >= 3 * n) return;
-    const int a = t / n, g = leafList[t - a * n];
+    const long tt = (long)blockIdx.x * BS + threadIdx.x, t = tt / kAdjLanes;
+    if (t >= 3L * n) return;
+    const int a = (int)(t / n), g = leafList[t - (long)a * n];
     const double ab = ubarMac[(size_t)a * c_G + g];
-    if (ab != 0.0) advVelDof(T, teDst, level, V, A, g, 0, a, dt, ab);
+    if (ab != 0.0) advVelDof(T, teDst, level, V, A, g, 0, a, dt, ab, (int)(tt % kAdjLanes));
 }
 
 // Half-tilt nodes among the velocity tilts are left to k_adj_adv_half: the
 // forward's half-tilt pass overwrites every slot k_adv_tilt wrote for them.
 __global__ void k_adj_adv_tilt(Topo T, const double* teDst, const uint8_t* level, Vel V, AdjMap A, const int* list,
                                int n, double dt, const double* ubarTilt, const uint8_t* inHalf) {
-    const int t = blockIdx.x * BS + threadIdx.x;
-    if (t >= 8 * n) return;
-    const int g = list[t >> 3], k = t & 7;
+    const long tt = (long)blockIdx.x * BS + threadIdx.x, t = tt / kAdjLanes;
+    if (t >= 8L * n) return;
+    const int g = list[t >> 3], k = (int)(t & 7);
     if (inHalf[g]) return;
     const double ab = ubarTilt[(size_t)k * c_G + g];
-    if (ab != 0.0) advVelDof(T, teDst, level, V, A, g, 1, k, dt, ab);
+    if (ab != 0.0) advVelDof(T, teDst, level, V, A, g, 1, k, dt, ab, (int)(tt % kAdjLanes));
 }
 
 __global__ void k_adj_adv_half(Topo T, const double* teDst, const uint8_t* level, Vel V, AdjMap A, const int* halfList,
                                int n, double dt, const double* ubarTilt) {
-    const long t = (long)blockIdx.x * BS + threadIdx.x;
+    const long tt = (long)blockIdx.x * BS + threadIdx.x, t = tt / kAdjLanes;
     if (t >= 5L * n) return;
     const int g = halfList[t / 5], i = (int)(t % 5);
     const int k = c_halfSlot[T.thd[g]][i];
     const double ab = ubarTilt[(size_t)k * c_G + g];
-    if (ab != 0.0) advVelDof(T, teDst, level, V, A, g, 2, i, dt, ab);
+    if (ab != 0.0) advVelDof(T, teDst, level, V, A, g, 2, i, dt, ab, (int)(tt % kAdjLanes));
 }
 
 // Entries an advection step writes (1) or carries over (0): MAC of leaves,
@@ -2668,28 +2677,26 @@ int AdvectDevice::diffAdjointAdvect(ProjectDevice& pd, double dt, std::string& e
     A.adj[2] = xDtilt;
     const double* d0c = scal_[0][cur_[0]][0].as<double>();
     const double* d0v = scal_[0][cur_[0]][1].as<double>();
-    const int BSA = 64;  // heavy lanes: small blocks spread them over the CUs
-    auto nbA = [&](long n) { return (int)((n + BSA - 1) / BSA); };
-    (void)nbA;
     const uint8_t* ih = static_cast<const uint8_t*>(inHalf_.p);
+    auto nbAdj = [](long n) { return nblocks(n * kAdjLanes); };
     if (nLeaf_)
-        k_adj_adv_scalar<<<nblocks(nLeaf_), BS, 0, stream_>>>(T, lev, V, A, leaf_.as<int>(), nLeaf_, 0, dt, d0c, d0v,
-                                                              a + 11 * G, xCell, xVert, nullptr);
+        k_adj_adv_scalar<<<nbAdj(nLeaf_), BS, 0, stream_>>>(T, lev, V, A, leaf_.as<int>(), nLeaf_, 0, dt, d0c, d0v,
+                                                            a + 11 * G, xCell, xVert, nullptr);
     if (nOpenTilt_)
-        k_adj_adv_scalar<<<nblocks(nOpenTilt_), BS, 0, stream_>>>(T, lev, V, A, openTilt_.as<int>(), nOpenTilt_, 1,
-                                                                  dt, d0c, d0v, a + 12 * G, xCell, xVert, ih);
+        k_adj_adv_scalar<<<nbAdj(nOpenTilt_), BS, 0, stream_>>>(T, lev, V, A, openTilt_.as<int>(), nOpenTilt_, 1, dt,
+                                                                d0c, d0v, a + 12 * G, xCell, xVert, ih);
     if (nHalf_)
-        k_adj_adv_scalar<<<nblocks(nHalf_), BS, 0, stream_>>>(T, lev, V, A, half_.as<int>(), nHalf_, 1, dt, d0c, d0v,
-                                                              a + 12 * G, xCell, xVert, nullptr);
+        k_adj_adv_scalar<<<nbAdj(nHalf_), BS, 0, stream_>>>(T, lev, V, A, half_.as<int>(), nHalf_, 1, dt, d0c, d0v,
+                                                            a + 12 * G, xCell, xVert, nullptr);
     if (nLeaf_)
-        k_adj_adv_mac<<<nblocks(3L * nLeaf_), BS, 0, stream_>>>(T, te_.as<double>(), lev, V, A, leaf_.as<int>(),
-                                                                nLeaf_, dt, a);
+        k_adj_adv_mac<<<nbAdj(3L * nLeaf_), BS, 0, stream_>>>(T, te_.as<double>(), lev, V, A, leaf_.as<int>(), nLeaf_,
+                                                              dt, a);
     if (nVelTilt_)
-        k_adj_adv_tilt<<<nblocks(8L * nVelTilt_), BS, 0, stream_>>>(T, te_.as<double>(), lev, V, A,
-                                                                     velTilt_.as<int>(), nVelTilt_, dt, a + 3 * G, ih);
+        k_adj_adv_tilt<<<nbAdj(8L * nVelTilt_), BS, 0, stream_>>>(T, te_.as<double>(), lev, V, A, velTilt_.as<int>(),
+                                                                  nVelTilt_, dt, a + 3 * G, ih);
     if (nHalf_)
-        k_adj_adv_half<<<nblocks(5L * nHalf_), BS, 0, stream_>>>(T, te_.as<double>(), lev, V, A, half_.as<int>(),
-                                                                 nHalf_, dt, a + 3 * G);
+        k_adj_adv_half<<<nbAdj(5L * nHalf_), BS, 0, stream_>>>(T, te_.as<double>(), lev, V, A, half_.as<int>(),
+                                                               nHalf_, dt, a + 3 * G);
     HIPCHK(hipGetLastError());
     return ASTG_OK;
 }
