@@ -270,6 +270,8 @@ private:
     TileView tileView() const;
     template <typename T>
     int tileCoef(std::string& err);
+    int ensureTileCoef64(std::string& err);
+    bool isTileKernel(const void* f) const;
     template <typename T>
     int launchTile(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm, double tolRel,
                    int phases, std::string& err);

@@ -1132,10 +1132,11 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
         levRange_[2 * L + 1] = lf.gStart[L] + lf.gRows[L];
     }
     // PCG work vectors: sweep-ordered (PS entries) unless the row order is kept
-    perm_ = !rowOrderForced_;
-    if (const char* g = getenv("ASTG_ROW_ORDER")) perm_ = perm_ && atoi(g) == 0;
+    const char* keep = getenv("ASTG_ROW_ORDER");
+    const bool keepRows = keep && atoi(keep) != 0;
+    perm_ = !rowOrderForced_ && !keepRows;
     // sweeps: in tiles where they fit; otherwise q levels per group
-    if (perm_ && !noTile_)
+    if (!keepRows && !noTile_)
         if (int rc = tileSetup(tiled_, err)) return rc;
     if (!tiled_) {
         layout(merge_, gateDist_, true, ls);
@@ -1295,7 +1296,7 @@ int PcgDevice::prepareSolve(std::string& err) {
 }
 
 bool PcgDevice::isSweepKernel(const void* f) const {
-    return f == (const void*)k_fwd<double> || f == (const void*)k_fwd<float> || f == (const void*)k_bwd_dot<double> ||
+    return isTileKernel(f) || f == (const void*)k_fwd<double> || f == (const void*)k_fwd<float> || f == (const void*)k_bwd_dot<double> ||
            f == (const void*)k_bwd_dot<float>;
 }
 
@@ -1554,9 +1555,8 @@ int PcgDevice::solveOnce(const astg_pcg_params& prm, astg_pcg_result& res, std::
     if (tiled_ && prm.precision == ASTG_PREC_FP64) {
         if (!tilesFit(tileSlots_, 8)) {
             if (int rc = dropTiles(err)) return rc;
-        } else if (!tileCoef64_) {
-            if (int rc = tileCoef<double>(err)) return rc;
-            tileCoef64_ = true;
+        } else if (int rc = ensureTileCoef64(err)) {
+            return rc;
         }
     }
     const int n = vlen(), gs = gs_;
@@ -1697,10 +1697,7 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
             err = "the FP64 sweeps of this ordering need a FP64 solve first";
             return ASTG_ERR_STATE;
         }
-        if (!tileCoef64_) {
-            if (int rc = tileCoef<double>(err)) return rc;
-            tileCoef64_ = true;
-        }
+        if (int rc = ensureTileCoef64(err)) return rc;
     }
     // one direction of a sweep
     auto sweep64 = [&](int dir) -> int {
@@ -1848,6 +1845,12 @@ int PcgDevice::sweepTimeline(int which, std::vector<long long>& t, std::vector<i
     return ASTG_OK;
 }
 
+template void PcgDevice::armSweeps<double>();
+template void PcgDevice::armSweeps<float>();
+template int PcgDevice::precondition<double>(const double*, const double*, double*, int, int, int, int, int, double,
+                                             std::string&);
+template int PcgDevice::precondition<float>(const float*, const float*, float*, int, int, int, int, int, double,
+                                            std::string&);
 template int PcgDevice::launchFwd<double>(const double*, const double*, int, int, int, int, int, double,
                                           std::string&);
 template int PcgDevice::launchFwd<float>(const float*, const float*, int, int, int, int, int, double, std::string&);

@@ -4,7 +4,7 @@
 // The systems are stacked into one block-diagonal matrix, every system's rows
 // padded with identity rows (zero right-hand side) to a multiple of 256, so
 // that every 256-row chunk belongs to one system. The pattern-only work
-// (dependency levels, factorisation plan, merged sweep stencils) and the
+// (dependency levels, factorisation plan, tiles or merged sweep stencils) and the
 // factorisation are PcgDevice's own on the stacked matrix. With no coupling
 // between the blocks, the MIC(0) factor of the stack is the stack of the
 // systems' factors and a row's dependency level is its level inside its own
@@ -270,11 +270,6 @@ __global__ void kb_zero_count(int* c) {
 __global__ void kb_zero64(int n, double* x) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) x[i] = 0.0;
 }
-template <typename T>
-__global__ void kb_fill_sent(T* p, long n) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) Sentinel<T>::storeSent(&p[i]);
-}
 inline int nblocks(long n) { return (int)((n + BS - 1) / BS); }
 
 }  // namespace
@@ -372,9 +367,8 @@ int PcgDevice::pcgBatchInner(const T* A, const T* invd, const T* b, double* x, i
     kb_zero_count<<<1, 64, 0, stream_>>>(V.ndone);
     kb_init<T, double><<<g, BS, 0, stream_>>>(V, b, x, r, norm);
     kb_reduce<<<V.K, BS, 0, stream_>>>(V, P_INIT, norm, scal);
-    kb_fill_sent<T><<<nblocks(2 * (long)PS_), BS, 0, stream_>>>(y_.as<T>(), 2 * (long)PS_);
-    if ((rc = launchFwd<T>(invd, r, 0, 2, 0, maxIt, norm, 0.0, err))) return rc;
-    if ((rc = launchBwd<T>(invd, r, z, 0, 0, err))) return rc;
+    armSweeps<T>();
+    if ((rc = precondition<T>(invd, r, z, 0, 2, 0, maxIt, norm, 0.0, err))) return rc;
     kb_dot<T><<<g, BS, 0, stream_>>>(V, z, r);
     kb_reduce<<<V.K, BS, 0, stream_>>>(V, P_RHO0, norm, scal);
     kb_xpby<T><<<g, BS, 0, stream_>>>(V, z, s, 0);
@@ -399,9 +393,7 @@ int PcgDevice::pcgBatchInner(const T* A, const T* invd, const T* b, double* x, i
                 kb_replace_res<8><<<g, BS, 0, stream_>>>(V, rs, col, val_.as<double>(), x, b64, r32, norm);
         }
         kb_reduce<<<V.K, BS, 0, stream_>>>(V, P_RES, norm, scal);
-        int e = launchFwd<T>(invd, r, itx + 1, 2, itx, maxIt, norm, 0.0, err);
-        if (!e) e = launchBwd<T>(invd, r, z, itx + 1, (itx + 1) & 1, err);
-        if (e) return e;
+        if (int e = precondition<T>(invd, r, z, itx + 1, 2, itx, maxIt, norm, 0.0, err)) return e;
         kb_dot<T><<<g, BS, 0, stream_>>>(V, z, r);
         kb_reduce<<<V.K, BS, 0, stream_>>>(V, P_RHO, norm, scal);
         kb_xpby<T><<<g, BS, 0, stream_>>>(V, z, s, 1);
@@ -521,6 +513,7 @@ int PcgDevice::solveBatchOnce(const astg_pcg_params& prm, std::vector<astg_pcg_r
     std::vector<double> st((size_t)K * B_COUNT, 0.0);
     auto S = [&](int k, int slot) -> double& { return st[(size_t)k * B_COUNT + slot]; };
     if (prm.precision == ASTG_PREC_FP64) {
+        if (int rc = ensureTileCoef64(err)) return rc;
         for (int k = 0; k < K; ++k) {
             S(k, B_TOLREL) = prm.tol;
             S(k, B_MAXIT) = maxIt;

@@ -334,15 +334,19 @@ __device__ inline void tile_export(const TileDir& D, const uint16_t* xslot, cons
     }
 }
 
+// Forms of the sweep: vectors by position; the same with a timeline of every
+// row; r, z and the pivots by row (batched solves).
+enum TileMode { kTilePlain, kTileTrace, kTileByRow };
+
 // A 64-row chunk's data in registers.
 template <typename T>
 struct TileChunk {
     Pair<T> f[kMaxDeps / 2];
     uint32_t sl[kMaxDeps / 2];
     T y, inv, r;
-    int step, w, t;
+    int step, w, t, v;  // v: the row (kTileByRow), -1 padding
 };
-template <typename T, int DIR>
+template <typename T, int DIR, int MODE>
 __device__ inline void tile_load(TileChunk<T>& C, const TileView& V, const Pair<T>* coef, const T* invd, const T* r,
                                  const T* y, int chunk, int base, int w) {
     const int lane = threadIdx.x & 63;
@@ -355,9 +359,18 @@ __device__ inline void tile_load(TileChunk<T>& C, const TileView& V, const Pair<
             C.sl[k] = V.d[DIR].slot[q + (size_t)k * 64];
             C.f[k] = coef[q + (size_t)k * 64];
         }
-    C.r = r[C.t];
+    if constexpr (MODE == kTileByRow) {
+        C.v = V.order[C.t];
+        C.r = C.inv = (T)0;  // padding: the row's value is zero
+        if (C.v >= 0) {
+            C.r = r[C.v];
+            C.inv = invd[C.v];
+        }
+    } else {
+        C.r = r[C.t];
+        C.inv = invd[C.t];
+    }
     if (DIR == 1) C.y = y[C.t];
-    C.inv = invd[C.t];
     C.step = V.step[C.t];
 }
 // The chunk's loads have arrived: waited for here, once, and not at their uses
@@ -432,7 +445,7 @@ __device__ inline bool tile_rows(const TileChunk<T>& C, T* lds, T* own, T& v, lo
 // reversed), every kTileWaves-th from the wavefront's own, so that a chunk's
 // data is loaded while the chunks before it are worked on. out: y or z; dot: the
 // backward sweep's z.r.
-template <typename T, int DIR, bool TRACE>
+template <typename T, int DIR, int MODE>
 __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const T* invd, const T* r, const T* y,
                                    T* out, double& dot, int p0, int wave, T* lds, long long t0, int* err, int bit) {
     const int chunks = V.S / 64, first = p0 / 64 + wave, count = (chunks - wave + kTileWaves - 1) / kTileWaves;
@@ -446,7 +459,7 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
     auto load = [&](TileChunk<T>& C, int j) {
         const int base = j < 64 ? __builtin_amdgcn_readlane(s0, j) : __builtin_amdgcn_readlane(s1, j - 64);
         const int end = j < 64 ? __builtin_amdgcn_readlane(e0, j) : __builtin_amdgcn_readlane(e1, j - 64);
-        tile_load<T, DIR>(C, V, coef, invd, r, y, chunk(j), base, end - base);
+        tile_load<T, DIR, MODE>(C, V, coef, invd, r, y, chunk(j), base, end - base);
     };
     auto work = [&](TileChunk<T>& C) {
         T v = (T)0;
@@ -454,7 +467,7 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
         T* own = &lds[C.t - p0];
         bool ok = false;
 #define ASTG_TILE_ROWS(W) \
-    case W: ok = tile_rows<T, DIR, W, TRACE>(C, lds, own, v, seen, t0, err, bit); break;
+    case W: ok = tile_rows<T, DIR, W, MODE == kTileTrace>(C, lds, own, v, seen, t0, err, bit); break;
         switch (C.w) {
             ASTG_TILE_ROWS(0)
             ASTG_TILE_ROWS(1)
@@ -468,9 +481,13 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
         }
 #undef ASTG_TILE_ROWS
         static_assert(kMaxDeps == 16, "one case per width");
-        out[C.t] = v;
+        if constexpr (DIR == 1 && MODE == kTileByRow) {
+            if (C.v >= 0) out[C.v] = v;
+        } else {
+            out[C.t] = v;
+        }
         if (DIR == 1) dot += (double)v * (double)C.r;
-        if (TRACE && V.order[C.t] >= 0) {
+        if (MODE == kTileTrace && V.order[C.t] >= 0) {
             long long* tr = V.trace + 3 * (long)V.order[C.t];
             tr[0] = t0;
             tr[1] = seen;
@@ -512,7 +529,7 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
 // those of the next one, armed here. A position is worked on by the
 // same lane in both sweeps, so y needs no hand-over.
 constexpr int kTileThreads = 64 * (kTileWaves + kTileImport + kTileExport);
-template <typename T, bool TRACE>
+template <typename T, int MODE>
 __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const Pair<T>* coefF, const Pair<T>* coefB,
                                                              const T* invd, const T* r, T* y, T* z, T* xF, T* xB,
                                                              T* nF, T* nB, Parts Pt, int* cnt, double* scal, int mode,
@@ -542,11 +559,11 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const P
     if (threadIdx.x == 0) lds[zero] = (T)0;
     if (phases & 1) {
         arm(V.d[0], nF);
-        if (fwd_prologue<NT>(Pt, scal, mode, it, maxIt, norm, tolRel)) return;
+        if (mode != 2 && fwd_prologue<NT>(Pt, scal, mode, it, maxIt, norm, tolRel)) return;
         __syncthreads();
         const long long t0 = wall_clock64();
         if (wave < kTileWaves)
-            tile_chunks<T, 0, TRACE>(V, coefF, invd, r, y, y, dot, p0, wave, lds, t0, err, E_FWD);
+            tile_chunks<T, 0, MODE>(V, coefF, invd, r, y, y, dot, p0, wave, lds, t0, err, E_FWD);
         else if (wave < kTileWaves + kTileImport)
             tile_import<T, 0>(V.d[0], p0, S, xF, lds + S, threadIdx.x - kTileWaves * 64, t0, err, E_FWD);
         else
@@ -559,7 +576,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const P
     __syncthreads();
     const long long t0 = wall_clock64();
     if (wave < kTileWaves)
-        tile_chunks<T, 1, TRACE>(V, coefB, invd, r, y, z, dot, p0, wave, lds, t0, err, E_BWD);
+        tile_chunks<T, 1, MODE>(V, coefB, invd, r, y, z, dot, p0, wave, lds, t0, err, E_BWD);
     else if (wave < kTileWaves + kTileImport)
         tile_import<T, 1>(V.d[1], p0, S, xB, lds + S, threadIdx.x - kTileWaves * 64, t0, err, E_BWD);
     else
@@ -599,7 +616,10 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
     used = false;
     const int n = n_;
     const bool placed = coordExt_[0] > 0;
-    int K = std::min(cus_, placed ? std::max(1, n / kTileRows) : (n + kTileRangeRows - 1) / kTileRangeRows);
+    // a batch's chains end at its systems' boundaries, so its ranges are half as long
+    // (6 systems of 12^3 to 56^3, FP32, ms per solve: 12 tiles 10.7, 16 9.7, 24 9.2, 48 9.6)
+    const int range = rowOrderForced_ ? kTileRangeRows / 2 : kTileRangeRows;
+    int K = std::min(cus_, placed ? std::max(1, n / kTileRows) : (n + range - 1) / range);
     if (const char* g = getenv("ASTG_TILES")) {
         if (atoi(g) <= 0) return ASTG_OK;
         K = std::min(atoi(g), cus_);
@@ -735,6 +755,7 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
     }
     HIPCHK(hipGetLastError());
     PS_ = P;
+    tileLds64_ = tileLds32_ = false;  // the form of the kernel may have changed
     used = true;
     return ASTG_OK;
 }
@@ -758,6 +779,19 @@ TileView PcgDevice::tileView() const {
     return v;
 }
 
+bool PcgDevice::isTileKernel(const void* f) const {
+    return f == (const void*)k_tile_sweep<double, kTilePlain> || f == (const void*)k_tile_sweep<float, kTilePlain> ||
+           f == (const void*)k_tile_sweep<double, kTileByRow> || f == (const void*)k_tile_sweep<float, kTileByRow>;
+}
+
+// FP64 solves: the coefficients of the current factor, gathered once per factor.
+int PcgDevice::ensureTileCoef64(std::string& err) {
+    if (!tiled_ || tileCoef64_) return ASTG_OK;
+    if (int rc = tileCoef<double>(err)) return rc;
+    tileCoef64_ = true;
+    return ASTG_OK;
+}
+
 template <typename T>
 int PcgDevice::tileCoef(std::string& err) {
     for (int d = 0; d < 2; ++d) {
@@ -774,7 +808,9 @@ int PcgDevice::tileCoef(std::string& err) {
 template <typename T>
 int PcgDevice::launchTile(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm,
                           double tolRel, int phases, std::string& err) {
-    const auto kernel = trace_ ? k_tile_sweep<T, true> : k_tile_sweep<T, false>;
+    const auto kernel = !perm_   ? k_tile_sweep<T, kTileByRow>
+                        : trace_ ? k_tile_sweep<T, kTileTrace>
+                                 : k_tile_sweep<T, kTilePlain>;
     const size_t lds = tileLds(tileSlots_, sizeof(T));
     bool& raised = sizeof(T) == 8 ? tileLds64_ : tileLds32_;
     if (!raised || trace_) {

@@ -116,3 +116,29 @@ def test_uniform_matches_merged_sweeps(res, precision, monkeypatch):
     for it, u in out[1:]:
         assert abs(it - out[0][0]) <= (1 if precision == "fp64" else 4)
         assert np.abs(u - out[0][1]).max() <= 1e-7 * np.abs(u).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("tiles", [1, 3, 16])
+def test_batch_matches_merged_sweeps(tiles, precision, monkeypatch):
+    """Stacked systems through tiles that cut them anywhere, and a system of a
+    single row among them."""
+    import astg
+    rng = np.random.default_rng(11)
+    systems = []
+    for shape in ((1, 1, 1), (9, 8, 7), (1, 20, 31), (16, 17, 18), (3, 3, 3)):
+        rs, col, val = box(shape, rng)
+        systems.append((rs, col, val, rng.standard_normal(len(rs) - 1)))
+    prm = astg.default_params(tol=1e-11, max_iterations=3000,
+                              precision=astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64)
+    out = []
+    for t in (0, tiles):
+        monkeypatch.setenv("ASTG_TILES", str(t))
+        c = astg.Context(0)
+        out.append(c.pcg_solve_batch(systems, prm))
+        c.close()
+    (x0, r0), (x1, r1) = out
+    for s, a, b, p, q in zip(systems, x0, x1, r0, r1):
+        assert p.converged and q.converged and abs(p.iterations - q.iterations) <= 2
+        # both within tol ||b|| / 0.05 of the solution (test_csr_matches_oracle)
+        assert np.abs(a - b).max() <= 2 * 1e-11 * np.abs(s[3]).max() / 0.05
