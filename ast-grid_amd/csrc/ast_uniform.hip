@@ -545,7 +545,8 @@ int AstUniform::ensurePattern(std::string& err) {
     return ASTG_OK;
 }
 
-// Block size in cells, and levels per sweep group of the block-colour solver:
+// Block size in cells, and levels per sweep group of the block-colour solver
+// where its sweeps are merged (the figures are the merged sweeps'):
 // pairs below a million rows (a few thousand rows per level, where the
 // substituted dependencies cost less than the dependent step they save),
 // single levels above. ASTG_AST_BLOCK / ASTG_AST_MERGE override them. Measured
@@ -558,7 +559,8 @@ static int astBlock() {
     const int v = e ? std::atoi(e) : 0;
     return v > 0 ? v : 4;
 }
-// Levels per sweep group of the reference-numbered solver: in 2D the levels
+// Levels per sweep group of the reference-numbered solver where its sweeps are
+// merged (systems too large for tiles): in 2D the levels
 // are a few hundred rows (the chain is nx + ny deep), so deep groups pay:
 // 192x384 FP64, ms per projection at 2 / 3 / 4 / 6 / 8 levels per group:
 // 342 / 235 / 180 / 136 / 133 (384x768: 1342 / - / 694 / 503 / 480), the same

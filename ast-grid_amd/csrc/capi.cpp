@@ -501,7 +501,7 @@ int astg_project(astg_ctx* c, double dt, double rho, const astg_pcg_params* para
 
 namespace {
 // Cube size of the block-colour ordering in finest cells, and the dependency
-// levels per sweep group of its solver (ASTG_BLOCK_CELLS / ASTG_BLOCK_MERGE
+// levels per sweep group of its solver where its sweeps are merged (ASTG_BLOCK_CELLS / ASTG_BLOCK_MERGE
 // override them for experiments). Measured at 256^3 (mixed form, ms per
 // projection): 8^3 cubes unmerged 164.8, 4^3 unmerged 173.0, 8^3 in level
 // pairs 188.9, 4^3 in pairs 180.9, 2^3 in pairs 234.7; with about 50 k rows
@@ -529,7 +529,7 @@ double micTau(const astg_pcg_params& prm) {
 
 // ASTG_ORDER_AUTO: the block-colour form for the mixed precision, the
 // reference numbering for FP64. The block-colour copy is built on the device
-// (C2: 26 ms against a 79 ms solve), so it pays from the first solve on a
+// (C2: 26 ms against a 58 ms solve), so it pays from the first solve on a
 // pattern, also in a run whose tilts change every step.
 bool blockOrdered(const astg_pcg_params& prm) {
     if (prm.ordering == ASTG_ORDER_BLOCK_COLOUR) return true;
