@@ -142,3 +142,37 @@ def test_batch_matches_merged_sweeps(tiles, precision, monkeypatch):
         assert p.converged and q.converged and abs(p.iterations - q.iterations) <= 2
         # both within tol ||b|| / 0.05 of the solution (test_csr_matches_oracle)
         assert np.abs(a - b).max() <= 2 * 1e-11 * np.abs(s[3]).max() / 0.05
+
+
+def test_fp64_solve_on_tiles_that_hold_fp32_only(monkeypatch):
+    """A block-colour pattern whose tiles fit the LDS in FP32 only: its first
+    FP64 solve rebuilds it with merged sweeps and gives what those give, and
+    the mixed form works before and after."""
+    import astg
+    from astg import scenes
+    fp64 = astg.default_params(tol=1e-10, max_iterations=3000, ordering=astg.ORDER_BLOCK_COLOUR)
+    mixed = astg.default_params(tol=1e-10, max_iterations=3000, precision=astg.PREC_MIXED)
+    out = []
+    for tiled in (False, True):
+        monkeypatch.setenv("ASTG_TILES", "0")
+        ctx, info = scenes.smoke_64(device=0, R=96)
+        scenes.fill_velocity(ctx, info["levels"], 3)
+        if tiled:
+            n = ctx.numbering(0)[2]
+            # 20 k to 40 k rows a tile: above 160 KB in FP64, below in FP32
+            monkeypatch.setenv("ASTG_TILES", str(max(1, round(n / 28000))))
+        ctx.snapshot(False)
+        m0 = ctx.project(info["dt"], info["rho"], mixed)
+        ctx.snapshot(True)
+        r = ctx.project(info["dt"], info["rho"], fp64)
+        p = ctx.system(r.n, r.nnz)[4]
+        ctx.snapshot(True)
+        m1 = ctx.project(info["dt"], info["rho"], mixed)
+        pm = ctx.system(r.n, r.nnz)[4]
+        assert m0.converged and r.converged and m1.converged
+        assert np.linalg.norm(pm - p) <= 2e-6 * np.linalg.norm(p)
+        out.append((r.n, r.iterations, p))
+        ctx.close()
+    (n, i0, p0), (_, i1, p1) = out
+    print("n %d" % n)
+    assert i0 == i1 and np.array_equal(p0, p1)
