@@ -353,8 +353,7 @@ template <typename T>
 __global__ void __launch_bounds__(BS) k_fwd(SweepPlan S, StencilView<T> St, const T* invd, const T* r, T* y, T* zp,
                                             Parts Pt, int* cnt, double* scal, int mode, int it, int maxIt, int norm,
                                             double tolRel) {
-    // a sweep of this solve already failed: the host retries the whole solve
-    if (scal[S_DONE] != 0.0 || ld_agent_i32(&cnt[C_ERR]) != 0) return;
+    if (sweep_stopped(scal, cnt)) return;
     if (mode != 2 && fwd_prologue(Pt, scal, mode, it, maxIt, norm, tolRel)) return;
     for (int c = blockIdx.x; c < S.nchunks; c += gridDim.x) {
         const int t = c * BS + threadIdx.x;
@@ -405,7 +404,7 @@ template <typename T>
 __global__ void __launch_bounds__(BS) k_bwd_dot(SweepPlan S, StencilView<T> St, const T* invd, const T* y, T* ynext,
                                                 const T* r, T* z, T* zp, Parts Pt, int* cnt, const double* scal,
                                                 int parityOut) {
-    if (scal[S_DONE] != 0.0 || ld_agent_i32(&cnt[C_ERR]) != 0) return;
+    if (sweep_stopped(scal, cnt)) return;
     double v = 0.0;
     for (int c = blockIdx.x; c < S.nchunks; c += gridDim.x) {
         const int pos = S.P - 1 - (c * BS + threadIdx.x);

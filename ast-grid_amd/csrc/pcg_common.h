@@ -48,6 +48,19 @@ __device__ inline double reduce_prev(const double* part, int np) {
     return block_reduce<MAX, NT>(acc);
 }
 
+// A sweep launch with nothing to do: the solve has stopped, or a sweep of it
+// failed (the host retries the whole solve). One thread looks, for its whole
+// block: in a launch whose first block stores S_DONE (fwd_prologue), or whose
+// rows raise an error bit, the wavefronts of a block that starts late could
+// otherwise find different values, and those that stay would reduce without
+// the partials of those that left.
+__device__ inline bool sweep_stopped(const double* scal, const int* cnt) {
+    __shared__ int stop;
+    if (threadIdx.x == 0) stop = scal[S_DONE] != 0.0 || ld_agent_i32(&cnt[C_ERR]) != 0;
+    __syncthreads();
+    return stop != 0;
+}
+
 // Forward sweep y = L^-1 r. mode 0 (start of the solve): ||b|| from the
 // partials, tolerance, zero-rhs exit. mode 1 (iteration `it`): the reference's
 // convergence test on the updated residual, before preconditioning. mode 2:

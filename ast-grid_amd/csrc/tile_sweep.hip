@@ -540,8 +540,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const P
     T* lds = reinterpret_cast<T*>(tile_lds);
     int* xdest = reinterpret_cast<int*>(lds + V.slots);
     uint16_t* xslot = reinterpret_cast<uint16_t*>(xdest + V.exports);
-    // a sweep of this solve already failed: the host retries the whole solve
-    if (scal[S_DONE] != 0.0 || ld_agent_i32(&cnt[C_ERR]) != 0) return;
+    if (sweep_stopped(scal, cnt)) return;
     const int S = V.S, p0 = blockIdx.x * S, zero = V.slots - 1;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int* err = &cnt[C_ERR];

@@ -176,3 +176,34 @@ def test_fp64_solve_on_tiles_that_hold_fp32_only(monkeypatch):
     (n, i0, p0), (_, i1, p1) = out
     print("n %d" % n)
     assert i0 == i1 and np.array_equal(p0, p1)
+
+
+@pytest.mark.parametrize("tiles", ["256", "0"], ids=["tiled", "merged"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_stopping_launch_ends_in_every_block(precision, tiles, monkeypatch, capfd):
+    """The launch that finds the solve finished stores that while its other
+    blocks start: each of them leaves as a whole or takes the decision itself.
+    Solves that end on many different launches, by convergence, by the
+    iteration limit and on a zero right-hand side: no block waits for one that
+    left (which would be reported and retried), and every repetition gives the
+    same solution."""
+    import astg
+    rng = np.random.default_rng(2)
+    rs, col, val = box((24, 25, 26), rng)
+    b = rng.standard_normal(len(rs) - 1)
+    prec = astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64
+    monkeypatch.setenv("ASTG_TILES", tiles)
+    c = astg.Context(0)
+    first = {}
+    for rep in range(6):
+        for tol, limit in [(10.0 ** -k, 3000) for k in range(1, 9)] + [(1e-9, k) for k in range(1, 9)]:
+            x, r = c.pcg_solve_csr(rs, col, val, b, astg.default_params(tol=tol, max_iterations=limit, precision=prec),
+                                   allow_unconverged=True)
+            key = tol, limit
+            if key not in first:
+                first[key] = x, r.iterations
+            assert r.iterations == first[key][1] and np.array_equal(x, first[key][0])
+        x, r = c.pcg_solve_csr(rs, col, val, 0 * b, astg.default_params(precision=prec))
+        assert r.iterations == 0 and not x.any()
+    c.close()
+    assert "retrying" not in capfd.readouterr().err
