@@ -265,6 +265,7 @@ private:
     // do not fit, the merged sweeps serve), their coefficients, one launch.
     int tileSetup(bool& used, std::string& err);
     int dropTiles(std::string& err);
+    int tileSystems(std::string& err);  // batched form: the system of every position
     bool tilesFit(int slots, int width) const;  // values of `width` bytes: the LDS holds them
     size_t tileLds(int slots, int width) const;
     TileView tileView() const;
@@ -360,7 +361,7 @@ private:
     int tileExports_ = 0;                   // longest export list of a tile
     int coordExt_[3] = {0, 0, 0};           // coordinate extents of rowCoord_ (0: none)
     DevTile tile_[2];
-    DevBuf rowCoord_, tileStep_;            // row positions; steps
+    DevBuf rowCoord_, tileStep_, tileSys_;  // row positions; steps and systems of the positions
     DevBuf tileKey_, tileKey2_, tileVal_, tileVal2_, tileOf_, tileCnt_, tileMax_, entryHalo_;  // set-up
     bool batchGraph_ = true;                // batched form: iterations replayed from hipGraphs
     bool coop_ = false;                     // sweeps through the cooperative launch API (ASTG_COOP=1)

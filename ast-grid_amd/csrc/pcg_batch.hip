@@ -300,7 +300,7 @@ int PcgDevice::setBatch(const std::vector<int>& segRow, std::string& err) {
     HIPCHK(hipMemcpyAsync(segChunk_.p, segChunk.data(), (size_t)(K + 1) * 4, hipMemcpyHostToDevice, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
     K_ = K;
-    return ASTG_OK;
+    return tiled_ ? tileSystems(err) : ASTG_OK;
 }
 
 int PcgDevice::batchGrid() const {

@@ -35,6 +35,10 @@ constexpr int kTileWaves = 12;
 constexpr int kTileImport = 2;
 constexpr int kTileExport = 2;
 
+// A system's state in the batched solves: 16 doubles (BatchSlot), looked at as
+// the upper words of the doubles.
+constexpr int kSysStride = 32;
+
 // One direction of the tiled sweeps (forward: lower entries, backward: upper).
 struct TileDir {
     const int* sell;       // per chunk: first entry pair (64 lanes each); nchunks + 1
@@ -49,6 +53,9 @@ struct TileView {
     TileDir d[2];
     const uint8_t* step;  // per position: the rank of its level among its chunk's levels
     const int* order;  // per position: row, -1 padding
+    const int* sys;    // batched solves, per position: the row's system
+    const int* sysDone;  // and per system, kSysStride apart: nonzero once it has finished
+    const int* ndone;    // and the number of systems that have
     int S;             // positions per tile
     int slots;         // LDS slots: S + H + 1
     int exports;       // room of the LDS export list

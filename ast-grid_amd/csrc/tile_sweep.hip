@@ -345,6 +345,7 @@ struct TileChunk {
     uint32_t sl[kMaxDeps / 2];
     T y, inv, r;
     int step, w, t, v;  // v: the row (kTileByRow), -1 padding
+    int done;           // the row's system has finished (kTileByRow)
 };
 template <typename T, int DIR, int MODE>
 __device__ inline void tile_load(TileChunk<T>& C, const TileView& V, const Pair<T>* coef, const T* invd, const T* r,
@@ -361,10 +362,14 @@ __device__ inline void tile_load(TileChunk<T>& C, const TileView& V, const Pair<
         }
     if constexpr (MODE == kTileByRow) {
         C.v = V.order[C.t];
+        const bool some = *V.ndone != 0;  // changes between launches only
+        const int s = some ? V.sys[C.t] : 0;
         C.r = C.inv = (T)0;  // padding: the row's value is zero
+        C.done = 0;
         if (C.v >= 0) {
             C.r = r[C.v];
             C.inv = invd[C.v];
+            if (some) C.done = V.sysDone[s * kSysStride];
         }
     } else {
         C.r = r[C.t];
@@ -390,13 +395,14 @@ __device__ inline void tile_arrived(TileChunk<T>& C) {
 // done unless they wait for another wavefront; it then looks again in every
 // round. A value not there yet is a NaN and makes the sum one, so the values
 // themselves are looked at only when the sum is a NaN. v: the row's value;
-// seen: the wall clock of its round (TRACE).
-template <typename T, int DIR, int W, bool TRACE>
+// seen: the wall clock of its round (kTileTrace).
+template <typename T, int DIR, int W, int MODE>
 __device__ inline bool tile_rows(const TileChunk<T>& C, T* lds, T* own, T& v, long long& seen, long long t0, int* err,
                                  int bit) {
     typedef typename Sentinel<T>::bits_t B;
     int step = C.step;
     if (DIR == 1) step = __shfl(step, 63, 64) - step;
+    if (MODE == kTileByRow && C.done) step = 0;
     const T* lo[W + 1];
     const T* hi[W + 1];
 #pragma unroll
@@ -428,7 +434,7 @@ __device__ inline bool tile_rows(const TileChunk<T>& C, T* lds, T* own, T& v, lo
             if (ready) {
                 v = a * C.inv;
                 lds_store<T>(own, to_bits(v));
-                if (TRACE) seen = wall_clock64();
+                if (MODE == kTileTrace) seen = wall_clock64();
                 pending = false;
             }
         }
@@ -450,6 +456,7 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
                                    T* out, double& dot, int p0, int wave, T* lds, long long t0, int* err, int bit) {
     const int chunks = V.S / 64, first = p0 / 64 + wave, count = (chunks - wave + kTileWaves - 1) / kTileWaves;
     if (count <= 0) return;
+    const int zero = V.slots - 1;
     // the chunks' entry starts and ends, in the lanes of four registers (count <= 128)
     const int lane = threadIdx.x & 63;
     auto chunk = [&](int j) { return first + kTileWaves * (DIR == 0 ? j : count - 1 - j); };
@@ -462,12 +469,27 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
         tile_load<T, DIR, MODE>(C, V, coef, invd, r, y, chunk(j), base, end - base);
     };
     auto work = [&](TileChunk<T>& C) {
+        if constexpr (MODE == kTileByRow) {
+            // a row of a finished system takes no part: a zero that waits for
+            // nothing (only its own system reads it). FP64 batches whose deepest
+            // system finishes in the first iterations, ms per solve without and
+            // with: a 20000-row chain and four 20^3 boxes 144 / 9.3, a 56^3 box and
+            // four red-black 20^3 boxes 10.3 / 4.7; six boxes that finish about
+            // together 9.31 / 9.32 (mixed).
+            if (C.done) {
+                C.v = -1;
+                C.r = C.inv = (T)0;
+                if (DIR == 1) C.y = (T)0;
+#pragma unroll
+                for (int k = 0; k < kMaxDeps / 2; ++k) C.sl[k] = (uint32_t)zero | (uint32_t)zero << 16;
+            }
+        }
         T v = (T)0;
         long long seen = 0;
         T* own = &lds[C.t - p0];
         bool ok = false;
 #define ASTG_TILE_ROWS(W) \
-    case W: ok = tile_rows<T, DIR, W, MODE == kTileTrace>(C, lds, own, v, seen, t0, err, bit); break;
+    case W: ok = tile_rows<T, DIR, W, MODE>(C, lds, own, v, seen, t0, err, bit); break;
         switch (C.w) {
             ASTG_TILE_ROWS(0)
             ASTG_TILE_ROWS(1)
@@ -610,6 +632,18 @@ bool PcgDevice::tilesFit(int slots, int width) const {
     return tileLds(slots, width) <= kTileLdsBytes;
 }
 size_t PcgDevice::tileLds(int slots, int width) const { return (size_t)slots * width + (size_t)tileExports_ * 6; }
+
+// The system of every position of the batched form's tiles (0 at padding).
+static __global__ void k_tile_sys(int P, const int* order, const int* chunkSeg, int* sys) {
+    const int t = blockIdx.x * BS + threadIdx.x;
+    if (t < P) sys[t] = order[t] >= 0 ? chunkSeg[order[t] / BS] : 0;
+}
+int PcgDevice::tileSystems(std::string& err) {
+    HIPCHK(tileSys_.alloc((size_t)PS_ * 4));
+    k_tile_sys<<<blocks(PS_), BS, 0, stream_>>>(PS_, sorder_.as<int>(), chunkSeg_.as<int>(), tileSys_.as<int>());
+    HIPCHK(hipGetLastError());
+    return ASTG_OK;
+}
 
 int PcgDevice::tileSetup(bool& used, std::string& err) {
     used = false;
@@ -771,6 +805,11 @@ TileView PcgDevice::tileView() const {
     }
     v.step = tileStep_.as<uint8_t>();
     v.order = sorder_.as<int>();
+    // the upper word of each system's B_DONE
+    static_assert(kSysStride == 2 * B_COUNT, "state of a system");
+    v.sys = K_ ? tileSys_.as<int>() : nullptr;
+    v.ndone = K_ ? bcnt_.as<int>() : nullptr;
+    v.sysDone = K_ ? bst_.as<int>() + 2 * B_DONE + 1 : nullptr;
     v.S = tileS_;
     v.slots = tileSlots_;
     v.exports = tileExports_;

@@ -207,3 +207,40 @@ def test_stopping_launch_ends_in_every_block(precision, tiles, monkeypatch, capf
         assert r.iterations == 0 and not x.any()
     c.close()
     assert "retrying" not in capfd.readouterr().err
+
+
+@pytest.mark.parametrize("tiles", [2, 5, 16])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_finished_systems_of_a_batch_take_no_part(precision, tiles, monkeypatch):
+    """The deepest system of the batch, a chain of 20000 rows whose factor is
+    exact, finishes first: the iterations after that do not run its chain. One
+    sweep over it takes at least 2 x 20000 dependent steps of over 0.1 us, so
+    the solve stays below half of iterations x 4 ms only without it. The
+    others' solutions are those they have without it in the batch."""
+    import astg
+    rng = np.random.default_rng(4)
+    others = []
+    for shape in ((20, 20, 20), (9, 8, 7), (1, 20, 31)):
+        rs, col, val = box(shape, rng)
+        others.append((rs, col, val, rng.standard_normal(len(rs) - 1)))
+    rs, col, val = box((1, 1, 20000), rng)
+    deep = (rs, col, val, rng.standard_normal(20000))
+    tol = 1e-11
+    prm = astg.default_params(tol=tol, max_iterations=3000,
+                              precision=astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64)
+    monkeypatch.setenv("ASTG_TILES", str(tiles))
+    c = astg.Context(0)
+    alone, ra = c.pcg_solve_batch(others, prm)
+    c.pcg_solve_batch([deep] + others, prm)  # plans and first launches
+    x, r = c.pcg_solve_batch([deep] + others, prm)
+    c.close()
+    most = max(q.iterations for q in r)
+    print("iterations %s, %.2f ms" % ([q.iterations for q in r], r[0].ms_solve))
+    assert r[0].iterations < most / 4
+    assert r[0].ms_solve < 0.5 * 4.0 * most
+    for s, u, v, p, q in zip(others, alone, x[1:], ra, r[1:]):
+        assert p.converged and q.converged and abs(p.iterations - q.iterations) <= 2
+        # both within tol ||b|| / 0.05 of the solution (test_csr_matches_oracle)
+        assert np.abs(u - v).max() <= 2 * tol * np.abs(s[3]).max() / 0.05
+    d = deep[2] * x[0][col]
+    assert np.abs(np.add.reduceat(d, rs[:-1]) - deep[3]).max() <= 2 * tol * np.abs(deep[3]).max()
