@@ -27,6 +27,21 @@ namespace {
 constexpr int kTileRows = 2048;
 constexpr int kTileRangeRows = 9600;
 
+// Index ranges cut an order of few wide levels (a colouring) everywhere: its
+// tiles import as many values as they hold rows, by 128 lanes, while merged
+// sweeps take it in a few steps over the whole chip. From 125 systems of boxes
+// and grids in ten orders, alone and in batches, FP64, ns per forward and
+// backward sweep: a level costs merged sweeps about 850 more than tiles, and the
+// second launch 8000; a tile costs 1.5 per row and 9 per imported value. us per
+// iteration tiled / merged: red-black 20^3 43 / 34, 2 x 30^3 in a batch 90 / 47;
+// blocks of 4 in 8 colours 28^3 83 / 69, 24 x 20^3 100 / 106, of 8 28^3 87 / 114;
+// natural order 28^3 80 / 161, 47 x 53 x 61 150 / 297; the form taken is at most
+// 9 % behind the other (one of the 250 in both precisions over 5 %). Boxes'
+// surfaces are small whatever the order: tiles cut by positions are not asked.
+inline bool rangesPay(int depth, int S, int halo) {
+    return 850ll * depth + 8000 >= 3ll * S / 2 + 9ll * halo;
+}
+
 inline int blocks(long n) { return (int)((n + BS - 1) / BS); }
 
 // ---------------------------------------------------------------------------
@@ -653,9 +668,10 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
     // (6 systems of 12^3 to 56^3, FP32, ms per solve: 12 tiles 10.7, 16 9.7, 24 9.2, 48 9.6)
     const int range = rowOrderForced_ ? kTileRangeRows / 2 : kTileRangeRows;
     int K = std::min(cus_, placed ? std::max(1, n / kTileRows) : (n + range - 1) / range);
-    if (const char* g = getenv("ASTG_TILES")) {
-        if (atoi(g) <= 0) return ASTG_OK;
-        K = std::min(atoi(g), cus_);
+    const char* forced = getenv("ASTG_TILES");
+    if (forced) {
+        if (atoi(forced) <= 0) return ASTG_OK;
+        K = std::min(atoi(forced), cus_);
     }
     int kk[3] = {1, 1, K};  // tiles per axis
     if (placed) {
@@ -766,6 +782,7 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
     // slots are named by 16 bits; the values and the export list share the LDS
     tileExports_ = h[5];
     if (slots > 65536 || !tilesFit((int)slots, tileFp32_ ? 4 : 8)) return ASTG_OK;
+    if (!placed && !forced && !rangesPay(depth_, S, h[4])) return ASTG_OK;
     tileK_ = K;
     tileS_ = S;
     tileSlots_ = (int)slots;

@@ -244,3 +244,52 @@ def test_finished_systems_of_a_batch_take_no_part(precision, tiles, monkeypatch)
         assert np.abs(u - v).max() <= 2 * tol * np.abs(s[3]).max() / 0.05
     d = deep[2] * x[0][col]
     assert np.abs(np.add.reduceat(d, rs[:-1]) - deep[3]).max() <= 2 * tol * np.abs(deep[3]).max()
+
+
+def ordered(rs, col, val, key):
+    """The matrix with its rows sorted by key."""
+    n = len(rs) - 1
+    new = np.empty(n, np.int64)
+    new[np.argsort(key, kind="stable")] = np.arange(n)
+    r, c = new[np.repeat(np.arange(n), np.diff(rs))], new[col]
+    o = np.lexsort((c, r))
+    return np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]).astype(np.int32), c[o].astype(np.int32), val[o]
+
+
+def colours(shape, blocks):
+    """0: none; 1: two colours; b: blocks of b cells in 8 colours."""
+    Z, Y, X = [a.ravel() for a in np.meshgrid(*[np.arange(s) for s in shape], indexing="ij")]
+    if blocks < 2:
+        return blocks * (X + Y + Z) % 2
+    x, y, z = X // blocks, Y // blocks, Z // blocks
+    return ((x & 1) + 2 * (y & 1) + 4 * (z & 1)) * 10 ** 6 + x + 100 * (y + 100 * z)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape,count,blocks,tiled", [
+    ((20, 20, 20), 1, 1, False), ((20, 20, 20), 1, 4, True), ((28, 28, 28), 1, 4, False), ((28, 28, 28), 1, 8, True),
+    ((28, 28, 28), 1, 0, True), ((20, 20, 20), 24, 1, False), ((30, 30, 30), 2, 4, False), ((30, 30, 30), 2, 0, True),
+])
+def test_orders_of_few_wide_levels_sweep_merged(shape, count, blocks, tiled, precision, monkeypatch):
+    """Index-range tiles are for long dependency chains; a colouring keeps the
+    merged sweeps. Which form a solve took shows in its solution's last bits."""
+    import astg
+    rng = np.random.default_rng(6)
+    systems = []
+    for _ in range(count):
+        rs, col, val = ordered(*box(shape, rng), colours(shape, blocks))
+        systems.append((rs, col, val, rng.standard_normal(len(rs) - 1)))
+    prm = astg.default_params(tol=1e-9, max_iterations=3000,
+                              precision=astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64)
+
+    def solve():
+        c = astg.Context(0)
+        x = c.pcg_solve_batch(systems, prm)[0] if count > 1 else [c.pcg_solve_csr(*systems[0], prm)[0]]
+        c.close()
+        return np.concatenate(x)
+
+    x = solve()
+    monkeypatch.setenv("ASTG_TILES", "0")
+    merged = solve()
+    assert np.array_equal(x, merged) == (not tiled)
+    assert np.abs(x - merged).max() <= 2 * 1e-9 * max(np.abs(s[3]).max() for s in systems) / 0.05
