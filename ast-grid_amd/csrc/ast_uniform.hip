@@ -525,7 +525,7 @@ int AstUniform::ensurePattern(std::string& err) {
     HIPCHK(hipGetLastError());
     pcg_.setMergeLevels(astRefMerge(g_.d));
     // rows' positions for the tiled sweeps (18 bits per axis; beyond, none)
-    coords_ = std::max({g_.res[0], g_.res[1], g_.d == 3 ? g_.res[2] : 0}) < (1 << 17);
+    coords_ = std::max({g_.res[0], g_.res[1], g_.d == 3 ? g_.res[2] : 0}) < (1 << 17) && PcgDevice::mayTile(n, 4);
     const int ext[3] = {2 * g_.res[0] + 1, 2 * g_.res[1] + 1, g_.d == 3 ? 2 * g_.res[2] + 1 : 1};
     if (coords_) {
         HIPCHK(coord_.alloc((size_t)n * 8));

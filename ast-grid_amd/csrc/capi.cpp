@@ -36,7 +36,7 @@ struct astg_ctx {
     std::unique_ptr<astg::PcgDevice> pcgBlk;              // the same system in block-colour order (reorder.h)
     astg::BlockOrderDevice blk;  // permutation and permuted pattern, device-built
     bool blkReady = false;
-    int coordExt[3] = {0, 0, 0};  // extents of the rows' positions (rowCoords)
+    int coordExt[3] = {0, 0, 0};  // extents of the rows' positions (rowCoords; 0: none)
     bool factoredBlk = false;  // the last factorisation was of the block-colour copy
     std::unique_ptr<astg::ProjectDevice> proj;
     std::unique_ptr<astg::AdvectDevice> adv;              // post-projection step and advection
@@ -78,11 +78,13 @@ int needDevice(astg_ctx* c) {
     return ASTG_OK;
 }
 
-// The projection system's pattern, with the rows' positions.
+// The projection system's pattern, with the rows' positions where a solver of
+// it can sweep in tiles (the block-colour copy's FP32 ones are the smallest).
 int setProjectionPattern(astg_ctx* c) {
     std::vector<unsigned long long> coord;
-    astg::rowCoords(*c->tree, c->num, coord, c->coordExt);
-    if (int rc = c->pcg->setCoords(c->tables.n, coord.data(), c->coordExt, c->err)) return rc;
+    c->coordExt[0] = 0;
+    if (astg::PcgDevice::mayTile(c->tables.n, 4)) astg::rowCoords(*c->tree, c->num, coord, c->coordExt);
+    if (int rc = c->pcg->setCoords(c->tables.n, coord.empty() ? nullptr : coord.data(), c->coordExt, c->err)) return rc;
     return c->pcg->setPattern(c->tables.n, c->tables.rowstart.data(), c->tables.col.data(), c->err);
 }
 
@@ -571,8 +573,10 @@ int ensureBlockOrder(astg_ctx* c) {
     if (!c->pcgBlk) c->pcgBlk.reset(new astg::PcgDevice(c->stream));
     c->pcgBlk->setMergeLevels(blockMerge());
     c->pcgBlk->setTileFp32(true);
-    if ((rc = c->pcgBlk->setCoordsDevice(n, c->pcg->devCoords(), c->blk.perm.as<int>(), c->coordExt, c->err)))
-        return rc;
+    rc = c->coordExt[0] > 0
+             ? c->pcgBlk->setCoordsDevice(n, c->pcg->devCoords(), c->blk.perm.as<int>(), c->coordExt, c->err)
+             : c->pcgBlk->setCoords(0, nullptr, nullptr, c->err);
+    if (rc) return rc;
     rc = c->pcgBlk->setPatternDevice(n, nnz, c->blk.rowstart.as<int>(), c->blk.col.as<int>(), c->err);
     if (rc) return rc;
     tm.mark("solver pattern");

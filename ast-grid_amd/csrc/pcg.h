@@ -203,6 +203,9 @@ public:
     // The same from device memory on this object's stream; row i is at
     // coord[perm[i]] (perm null: coord[i]).
     int setCoordsDevice(int n, const unsigned long long* coord, const int* perm, const int* ext, std::string& err);
+    // The values of n rows, `width` bytes each, fit the LDS of all compute units:
+    // without that no system of n rows sweeps in tiles, with any positions.
+    static bool mayTile(long long n, int width);
     const unsigned long long* devCoords() const { return rowCoord_.as<unsigned long long>(); }
     // Tiles whose values fit the LDS in FP32 only are taken too: for a pattern
     // whose solves are the mixed form's (an FP64 solve then rebuilds it).

@@ -660,6 +660,14 @@ int PcgDevice::tileSystems(std::string& err) {
     return ASTG_OK;
 }
 
+bool PcgDevice::mayTile(long long n, int width) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return true;
+    return (n + cus - 1) / std::max(1, cus) * width <= (long long)kTileLdsBytes;
+}
+
 int PcgDevice::tileSetup(bool& used, std::string& err) {
     used = false;
     const int n = n_;
@@ -679,8 +687,11 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
         K = kk[0] * kk[1] * kk[2];
     }
     if (K > n) return ASTG_OK;
+    const int width = tileFp32_ ? 4 : 8;  // of the values the tiles have to hold
     const long long S64 = (((long long)n + K - 1) / K + 63) / 64 * 64;
-    if (S64 >= 65535 || ((long long)K * depth_ << kWidthBits) >= (1ll << 32) || S64 * K >= (1ll << 31) - 64)
+    // rows alone that do not fit: nothing is set up
+    if (S64 >= 65535 || S64 * width > (long long)kTileLdsBytes || ((long long)K * depth_ << kWidthBits) >= (1ll << 32) ||
+        S64 * K >= (1ll << 31) - 64)
         return ASTG_OK;
     const int S = (int)S64, P = K * S, nch = P / 64;
     const size_t n4 = (size_t)n * 4, P4 = (size_t)P * 4;
@@ -781,7 +792,7 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
                 (long long)h[3] * 128);
     // slots are named by 16 bits; the values and the export list share the LDS
     tileExports_ = h[5];
-    if (slots > 65536 || !tilesFit((int)slots, tileFp32_ ? 4 : 8)) return ASTG_OK;
+    if (slots > 65536 || !tilesFit((int)slots, width)) return ASTG_OK;
     if (!placed && !forced && !rangesPay(depth_, S, h[4])) return ASTG_OK;
     tileK_ = K;
     tileS_ = S;

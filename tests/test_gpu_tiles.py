@@ -293,3 +293,20 @@ def test_orders_of_few_wide_levels_sweep_merged(shape, count, blocks, tiled, pre
     merged = solve()
     assert np.array_equal(x, merged) == (not tiled)
     assert np.abs(x - merged).max() <= 2 * 1e-9 * max(np.abs(s[3]).max() for s in systems) / 0.05
+
+
+@pytest.mark.parametrize("tiles,done", [(1, False), (2, True)])
+def test_no_tiles_are_set_up_for_rows_that_do_not_fit(tiles, done, monkeypatch, capfd):
+    """24000 rows in one tile exceed the LDS by their values alone: the set-up
+    (sorts, counts) is not begun. In two tiles they fit."""
+    import astg
+    rng = np.random.default_rng(8)
+    rs, col, val = box((20, 30, 40), rng)
+    b = rng.standard_normal(len(rs) - 1)
+    monkeypatch.setenv("ASTG_TILES", str(tiles))
+    monkeypatch.setenv("ASTG_TIMING", "1")
+    c = astg.Context(0)
+    x, r = c.pcg_solve_csr(rs, col, val, b, astg.default_params(tol=1e-8, max_iterations=3000))
+    c.close()
+    assert r.converged == 1
+    assert ("tiles: n 24000 " in capfd.readouterr().err) == done
