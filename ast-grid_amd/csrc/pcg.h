@@ -7,11 +7,12 @@
 //     sync-free pass;
 //   * the factorisation is level-synchronous (one launch per level, one row per
 //     lane, left-looking per row with the reference's accumulation order);
-//   * the triangular sweeps run in spatial tiles, one workgroup each, whose
-//     rows' values live in LDS (tile_sweep.h); systems too large for that, and
-//     batches, take sync-free persistent kernels over merged stencils
-//     (sweep_merge.h): each row publishes its value with an agent-scope atomic
-//     store over a signalling-NaN sentinel that dependants poll;
+//   * the triangular sweeps run in tiles, one workgroup each, whose rows' values
+//     live in LDS (tile_sweep.h); systems too large for that, and those of few
+//     wide levels without positions, take sync-free persistent kernels over
+//     merged stencils (sweep_merge.h): each row publishes its value with an
+//     agent-scope atomic store over a signalling-NaN sentinel that dependants
+//     poll;
 //   * dots, axpys and the convergence test are fused into the SpMV / update /
 //     sweep kernels with wave64 reductions; scalars stay on the device.
 #pragma once
@@ -28,6 +29,7 @@
 
 namespace astg {
 class PhaseTimer;
+struct LevelLayout;
 
 // Device allocations made through DevBuf so far in this process, and the
 // time spent in them (hipFree of the old buffer included).
@@ -104,6 +106,30 @@ struct DevTile {
     int halo = 0;     // halo entries of all tiles
 };
 
+// The sweeps of a pattern in one form, and what is stored in its order of the
+// rows: tiles, or merged stencils. Built by the first solve that takes it.
+struct SweepForm {
+    bool ready = false;      // built for the current pattern
+    bool tiled = false;
+    bool coef64 = false;     // the FP64 coefficients match the factor
+    bool f32 = false;        // the FP32 copies match the factor
+    int PS = 0;              // padded length of the sweep order
+    int gF64 = 0, gB64 = 0, gF32 = 0, gB32 = 0;  // persistent grids
+    DevBuf sorder;           // per position: row, -1 padding
+    DevBuf pos;              // row -> position
+    DevBuf prs, pcol, pmap;  // CSR in sweep order: rowstart, columns as positions, source entry
+    DevBuf valP, invdP, bP, xP;  // values, pivots, rhs and solution in sweep order
+    DevBuf val32, invd32;    // FP32 copies for the mixed form
+    // merged sweeps: gates, forward / backward stencils
+    DevBuf sgateF, sgateB;
+    DevStencil stF, stB;
+    // tiles
+    int tileK = 0, tileS = 0, tileSlots = 0;
+    int tileExports = 0;     // longest export list of a tile
+    DevTile tile[2];
+    DevBuf tileStep, tileSys;  // steps and systems of the positions
+};
+
 // Per-block partials of the reductions, consumed by the next kernel.
 struct Parts {
     double* sq;    // gs partials of s.q
@@ -145,11 +171,11 @@ public:
     explicit PcgDevice(hipStream_t s) : stream_(s) {}
     ~PcgDevice();
 
-    // Uploads a CSR pattern (host arrays) and builds everything that depends on
-    // the pattern only, on the device: diagonal / upper split, transpose map
-    // and structural checks, dependency levels, the padded level and sweep
-    // orders, the symbolic plans and, for single-system solves, A's pattern
-    // permuted to sweep order.
+    // Uploads a CSR pattern (host arrays) and builds what the factorisation
+    // needs of it, on the device: diagonal / upper split, transpose map and
+    // structural checks, dependency levels, the padded level order and the
+    // factorisation programs. The sweeps (SweepForm) are set up by the first
+    // solve that needs them: which form serves depends on the precision.
     int setPattern(int n, const int* rowstart, const int* col, std::string& err);
     // The same from a pattern already in device memory (rowstart n+1, col
     // nnz, on this object's stream): no host copy is made until one is needed.
@@ -207,8 +233,8 @@ public:
     // without that no system of n rows sweeps in tiles, with any positions.
     static bool mayTile(long long n, int width);
     const unsigned long long* devCoords() const { return rowCoord_.as<unsigned long long>(); }
-    // Tiles whose values fit the LDS in FP32 only are taken too: for a pattern
-    // whose solves are the mixed form's (an FP64 solve then rebuilds it).
+    // The mixed form also takes tiles whose values fit the LDS in FP32 only;
+    // FP64 solves on such a pattern have merged sweeps of their own beside them.
     void setTileFp32(bool on) { tileFp32_ = on; }
     // Levels per merged sweep group used by the next setPattern (0: default).
     void setMergeLevels(int q) { mergeLevels_ = q; }
@@ -246,35 +272,46 @@ private:
     // After a spin-limit failure under ordinary sweep launches: cooperative
     // launches from now on, error bits cleared; true if the solve should be retried.
     bool fallBackToCooperative(std::string& err);
-    // symbolic plans (factorisation programs, both merged stencils) built on
+    // symbolic plans (factorisation programs; both merged stencils) built on
     // the device from the uploaded pattern and sweep order (plan_device.hip);
     // the host planners serve when hostPlan_ is set
-    int planDevice(int maxY, bool stencils, std::string& err);
+    int planMicDevice(std::string& err);
+    int planStencilsDevice(int maxY, std::string& err);
+    // The sweep form of a precision becomes the current one (f_), built if the
+    // pattern has none yet.
+    int useForm(int precision, std::string& err);
+    int buildForm(SweepForm& f, int width, bool tryTiles, bool orMerged, std::string& err);
+    int mergedSetup(std::string& err);
+    hipError_t upload(DevBuf& d, const void* src, size_t bytes);
+    int scatterLevels(const LevelLayout& o, int q, DevBuf& ord, std::string& err);
+    int checkOrder(const LevelLayout& o, int q, int dist, bool gates, const DevBuf& ord, std::vector<int>& padded,
+                   const char* what, std::string& err);
+    int formVectors(std::string& err);
+    int ensureCoef64(std::string& err);
     // Sweep-ordered solve: permuted CSR, forward r-term keys as positions
-    // (once per pattern); values, pivots and rhs gathered per solve.
+    // (once per form); values, pivots and rhs gathered per solve.
     int permuteSetup(std::string& err);
     int prepareSolve(std::string& err);
-    int vlen() const { return perm_ ? PS_ : n_; }  // length of the PCG vectors
-    const int* sRs() const { return perm_ ? prs_.as<int>() : rs_.as<int>(); }
-    const int* sCol() const { return perm_ ? pcol_.as<int>() : col_.as<int>(); }
-    double* sVal64() const { return perm_ ? valP_.as<double>() : val_.as<double>(); }
-    double* sInvd64() const { return perm_ ? invdP_.as<double>() : invd_.as<double>(); }
-    double* sB() const { return perm_ ? bP_.as<double>() : b_.as<double>(); }
-    double* sX() const { return perm_ ? xP_.as<double>() : x_.as<double>(); }
+    int vlen() const { return perm_ ? f_->PS : n_; }  // length of the PCG vectors
+    const int* sRs() const { return perm_ ? f_->prs.as<int>() : rs_.as<int>(); }
+    const int* sCol() const { return perm_ ? f_->pcol.as<int>() : col_.as<int>(); }
+    double* sVal64() const { return perm_ ? f_->valP.as<double>() : val_.as<double>(); }
+    double* sInvd64() const { return perm_ ? f_->invdP.as<double>() : invd_.as<double>(); }
+    double* sB() const { return perm_ ? f_->bP.as<double>() : b_.as<double>(); }
+    double* sX() const { return perm_ ? f_->xP.as<double>() : x_.as<double>(); }
     template <typename T>
     void launchSpmv(int n, const int* rs, const int* col, const T* A, const T* s, T* q, const Parts& Pt,
                     const double* scal);
-    // Tiled sweeps (tile_sweep.hip): the tiles of the pattern (used false: they
-    // do not fit, the merged sweeps serve), their coefficients, one launch.
-    int tileSetup(bool& used, std::string& err);
-    int dropTiles(std::string& err);
+    // Tiled sweeps (tile_sweep.hip): the tiles of the pattern for values of
+    // `width` bytes (used false: they do not fit, or do not pay), their
+    // coefficients, one launch.
+    int tileSetup(int width, bool& used, std::string& err);
     int tileSystems(std::string& err);  // batched form: the system of every position
-    bool tilesFit(int slots, int width) const;  // values of `width` bytes: the LDS holds them
-    size_t tileLds(int slots, int width) const;
+    bool tilesFit(int width) const;  // values of `width` bytes: the LDS holds them
+    size_t tileLds(int width) const;
     TileView tileView() const;
     template <typename T>
     int tileCoef(std::string& err);
-    int ensureTileCoef64(std::string& err);
     bool isTileKernel(const void* f) const;
     template <typename T>
     int launchTile(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm, double tolRel,
@@ -291,13 +328,13 @@ private:
     template <typename T>
     StencilView<T> view(const DevStencil& s) const;
     template <typename T>
-    T* ybuf(int k) const { return y_.as<T>() + (size_t)(k & 1) * PS_; }
+    T* ybuf(int k) const { return y_.as<T>() + (size_t)(k & 1) * f_->PS; }
     int syncScalars(std::string& err);
     int checkErrors(const char* where, std::string& err);
     template <typename T>
-    int fwdGrid() const { return sizeof(T) == 8 ? gF64_ : gF32_; }
+    int fwdGrid() const { return sizeof(T) == 8 ? f_->gF64 : f_->gF32; }
     template <typename T>
-    int bwdGrid() const { return sizeof(T) == 8 ? gB64_ : gB32_; }
+    int bwdGrid() const { return sizeof(T) == 8 ? f_->gB64 : f_->gB32; }
     SweepPlan splan() const;  // sweeps: rows in super-level order
     Parts parts(int gb) const;
 
@@ -311,12 +348,16 @@ private:
     int setPatternImpl(int n, long long nnz, const int* dRowstart, const int* dCol, PhaseTimer& tm,
                        std::string& err);
     DevBuf rs_, col_, lend_, ubeg_, tpos_, order_, lev_;  // pattern split, level order (factorisation)
+    std::vector<int> hlvlStart_;           // first sorted row of each level, and n
     std::vector<int> levRange_;             // per level: [first, last + 1) position in the level order
     DevBuf micStart_, micProg_, live_;      // factorisation programs (mic_plan.h), eliminated columns
-    DevBuf sorder_, sgateF_, sgateB_;       // sweep order (super-levels) and its gates
-    DevStencil stF_, stB_;                  // merged forward / backward stencils
+    // [0]: the sweeps of FP64 solves, and of mixed ones unless [1] is ready; [1]: tiles that
+    // fit the LDS in FP32 only (setTileFp32)
+    SweepForm form_[2];
+    SweepForm* f_ = &form_[0];              // the form of the current solve
+    bool patternSet_ = false;               // the pattern's set-up is complete
+    bool narrowTried_ = false;              // whether [1] exists is known
     DevBuf val_, F_, invd_;                 // FP64 A, factor (symmetric copy), 1/pivot
-    DevBuf val32_, invd32_;                 // FP32 copies for the mixed form
     DevBuf b_, x_;                          // FP64 rhs / solution
     DevBuf r_, z_, s_, q_;                  // work vectors, vlen() entries (sized for FP64; reused as FP32)
     DevBuf y_, zp_;                         // sweep vectors in sweep order (2 x PS and PS)
@@ -330,12 +371,10 @@ private:
     DevBuf lvlStart_, grpStart_, grpFirst_; // set-up: first sorted row of each level; group layout of an order
     DevBuf planLen_, planPos_, planCnt_, planTmp_;  // set-up: plan counts, sweep positions, scan scratch
     int P_ = 0;                             // padded length of the level order
-    int PS_ = 0;                            // padded length of the sweep order
     int merge_ = 2;                         // levels per super-level of the sweeps
     int cus_ = 0;                           // compute units
     int gs_ = 0;                            // grid of the streaming kernels
     int gb_ = 0;                            // largest backward-sweep grid (rho partial slots)
-    int gF64_ = 0, gB64_ = 0, gF32_ = 0, gB32_ = 0;  // persistent grids
     int gateDist_ = 2;                      // sweep gates: groups back (forward) / ahead
     int pollCap_ = 1;
     int gateCap_ = 8;
@@ -350,27 +389,20 @@ private:
     int spmvLpr_ = 4;                       // ASTG_SPMV_LPR: lanes per row of the single-system SpMV
     int spmvRows_ = 2;                      // ASTG_SPMV_ROWS: rows in flight per lane group (1, 2 or 4; 4 lanes per row)
     bool rowOrderForced_ = false;           // setRowOrder (batched form)
-    DevBuf pos_;                            // row -> sweep position
-    DevBuf prs_, pcol_, pmap_;              // CSR in sweep order: rowstart, columns as positions, source entry
-    DevBuf valP_, invdP_, bP_, xP_;         // values, pivots, rhs and solution in sweep order
     DevBuf permLen_;                        // set-up: row lengths in sweep order
     // tiled sweeps
-    bool tiled_ = false;                    // the current pattern sweeps in tiles
-    bool noTile_ = false;                   // dropTiles: this set-up takes the merged sweeps
     bool tileFp32_ = false;                 // setTileFp32
-    bool tileCoef64_ = false;               // FP64 tile coefficients match the factor
-    bool tileLds64_ = false, tileLds32_ = false;  // dynamic LDS limit raised
-    int tileK_ = 0, tileS_ = 0, tileSlots_ = 0;
-    int tileExports_ = 0;                   // longest export list of a tile
+    bool tileLds_[2][3] = {};               // dynamic LDS limit raised, per kernel (precision, TileMode)
+    int tilesAsked_ = -1;                   // ASTG_TILES (-1: not set)
+    bool keepRows_ = false;                 // ASTG_ROW_ORDER
     int coordExt_[3] = {0, 0, 0};           // coordinate extents of rowCoord_ (0: none)
-    DevTile tile_[2];
-    DevBuf rowCoord_, tileStep_, tileSys_;  // row positions; steps and systems of the positions
+    int coordN_ = 0;                        // rows of rowCoord_
+    DevBuf rowCoord_;                       // row positions
     DevBuf tileKey_, tileKey2_, tileVal_, tileVal2_, tileOf_, tileCnt_, tileMax_, entryHalo_;  // set-up
     bool batchGraph_ = true;                // batched form: iterations replayed from hipGraphs
     bool coop_ = false;                     // sweeps through the cooperative launch API (ASTG_COOP=1)
     bool spinFailed_ = false;               // a sweep hit its spin limit since the last solve started
     bool forceSpinError_ = false;           // test hook (ASTG_TEST_SPIN_ERROR_ONCE): one forced spin error
-    bool f32Valid_ = false;                 // FP32 copies match the current factor (convert32 since factor)
 };
 
 }  // namespace astg

@@ -871,12 +871,98 @@ __global__ void k_gather_coord(int n, const unsigned long long* coord, const int
     if (i < n) out[i] = coord[perm ? perm[i] : i];
 }
 
+// Orders: rows in order of groups of q consecutive levels, every group
+// padded to a multiple of 64 rows so that a wavefront never holds rows of
+// two groups, the whole padded to a multiple of BS; gate rows: for each
+// 64-row segment of group G, one row of group G-dist (forward) and one of
+// group G+dist (backward), spread over that group. Every level 0..depth-1
+// holds at least one row, so every group is non-empty. The group layout
+// follows from the first sorted row of each level (lvlStart, depth+1
+// entries): computed on the host from that, rows scattered on the device.
+struct LevelLayout {
+    int ng = 0, P = 0;
+    std::vector<int> gStart, gFirst, gRows, gF, gB;
+};
+static LevelLayout levelLayout(const std::vector<int>& lvlStart, int q, int dist, bool gates) {
+    LevelLayout o;
+    const int depth = (int)lvlStart.size() - 1;
+    o.ng = (depth + q - 1) / q;
+    o.gStart.assign(o.ng, 0);
+    o.gFirst.assign(o.ng, 0);
+    o.gRows.assign(o.ng, 0);
+    long long pos = 0;
+    for (int G = 0; G < o.ng; ++G) {
+        const int first = lvlStart[G * q], end = lvlStart[std::min((G + 1) * q, depth)];
+        o.gFirst[G] = first;
+        o.gRows[G] = end - first;
+        o.gStart[G] = (int)pos;
+        pos = (pos + o.gRows[G] + 63) / 64 * 64;
+    }
+    pos = (pos + BS - 1) / BS * BS;
+    o.P = (int)pos;
+    if (!gates) return o;
+    const int nseg = o.P / 64;
+    o.gF.assign(nseg, -1);
+    o.gB.assign(nseg, -1);
+    std::vector<int> segG(nseg, -1);
+    for (int G = 0; G < o.ng; ++G) {
+        const int s0 = o.gStart[G] / 64, s1 = (o.gStart[G] + o.gRows[G] + 63) / 64;
+        for (int sg = s0; sg < s1; ++sg) segG[sg] = G;
+    }
+    for (int sg = 0; sg < nseg; ++sg) {
+        const int G = segG[sg];
+        if (G < 0) continue;
+        const unsigned h = (unsigned)sg * 2654435761u;
+        const int gf = G - dist, gb = G + dist;
+        if (gf >= 0) o.gF[sg] = o.gStart[gf] + (int)(h % (unsigned)o.gRows[gf]);
+        if (gb < o.ng) o.gB[sg] = o.gStart[gb] + (int)(h % (unsigned)o.gRows[gb]);
+    }
+    return o;
+}
+
+// Host array to the device; the source lives until the stream is synchronised.
+hipError_t PcgDevice::upload(DevBuf& d, const void* src, size_t bytes) {
+    hipError_t e = d.alloc(bytes);
+    if (e != hipSuccess) return e;
+    return hipMemcpyAsync(d.p, src, bytes, hipMemcpyHostToDevice, stream_);
+}
+
+int PcgDevice::scatterLevels(const LevelLayout& o, int q, DevBuf& ord, std::string& err) {
+    HIPCHK(upload(grpStart_, o.gStart.data(), (size_t)o.ng * 4));
+    HIPCHK(upload(grpFirst_, o.gFirst.data(), (size_t)o.ng * 4));
+    HIPCHK(ord.alloc((size_t)o.P * 4));
+    k_fill_i32<<<blocks(o.P), BS, 0, stream_>>>(ord.as<int>(), -1, o.P);
+    k_pad_order<<<blocks(n_), BS, 0, stream_>>>(n_, sortKeys_.as<int>(), sortRows_.as<int>(), q, grpStart_.as<int>(),
+                                               grpFirst_.as<int>(), ord.as<int>());
+    HIPCHK(hipGetLastError());
+    // the small group arrays are reused by the next call: finish this one
+    HIPCHK(hipStreamSynchronize(stream_));
+    return ASTG_OK;
+}
+
+// The device-built order `ord` of layout `o` against the host construction.
+int PcgDevice::checkOrder(const LevelLayout& o, int q, int dist, bool gates, const DevBuf& ord,
+                          std::vector<int>& padded, const char* what, std::string& err) {
+    std::vector<int> lev(n_), row(n_), gF, gB, dev(o.P);
+    HIPCHK(hipMemcpyAsync(lev.data(), sortKeys_.p, (size_t)n_ * 4, hipMemcpyDeviceToHost, stream_));
+    HIPCHK(hipMemcpyAsync(row.data(), sortRows_.p, (size_t)n_ * 4, hipMemcpyDeviceToHost, stream_));
+    HIPCHK(hipMemcpyAsync(dev.data(), ord.p, (size_t)o.P * 4, hipMemcpyDeviceToHost, stream_));
+    HIPCHK(hipStreamSynchronize(stream_));
+    hostOrder(q, dist, n_, depth_, lev, row, padded, gF, gB);
+    if ((int)padded.size() != o.P || padded != dev || (gates && (gF != o.gF || gB != o.gB))) {
+        err = std::string("device-built ") + what + " differs from the host construction";
+        return ASTG_ERR_HIP;
+    }
+    return ASTG_OK;
+}
+
 int PcgDevice::setCoords(int n, const unsigned long long* coord, const int* ext, std::string& err) {
     coordExt_[0] = 0;
     if (!coord) return ASTG_OK;
     HIPCHK(rowCoord_.alloc((size_t)n * 8));
     HIPCHK(hipMemcpyAsync(rowCoord_.p, coord, (size_t)n * 8, hipMemcpyHostToDevice, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
+    coordN_ = n;
     for (int a = 0; a < 3; ++a) coordExt_[a] = ext[a];
     return ASTG_OK;
 }
@@ -887,6 +973,7 @@ int PcgDevice::setCoordsDevice(int n, const unsigned long long* coord, const int
     HIPCHK(rowCoord_.alloc((size_t)n * 8));
     k_gather_coord<<<blocks(n), BS, 0, stream_>>>(n, coord, perm, rowCoord_.as<unsigned long long>());
     HIPCHK(hipGetLastError());
+    coordN_ = n;
     for (int a = 0; a < 3; ++a) coordExt_[a] = ext[a];
     return ASTG_OK;
 }
@@ -935,9 +1022,10 @@ int PcgDevice::ensureHostPattern(std::string& err) {
 // The pattern is in hrs_ / hcol_ (dRowstart null) or in device memory.
 int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const int* dCol, PhaseTimer& tm,
                               std::string& err) {
-    f32Valid_ = false;
-    tileCoef64_ = false;
-    tiled_ = false;
+    patternSet_ = false;
+    for (SweepForm& f : form_) f.ready = false;
+    f_ = &form_[0];
+    narrowTried_ = false;
     n_ = n;
     nnz_ = nnz;
     if (const char* g = getenv("ASTG_GATE_DIST")) gateDist_ = std::max(1, atoi(g));
@@ -984,9 +1072,7 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
     HIPCHK(cnt_.alloc(C_COUNT * 4));
     if (!hscal_) HIPCHK(hipHostMalloc((void**)&hscal_, 32 * 8, hipHostMallocDefault));
     if (!hplan_) HIPCHK(hipHostMalloc((void**)&hplan_, 16 * 8, hipHostMallocDefault));
-    if (dRowstart == rs_.p) {
-        // the pattern is in place (dropTiles)
-    } else if (dRowstart) {
+    if (dRowstart) {
         HIPCHK(hipMemcpyAsync(rs_.p, dRowstart, ((size_t)n + 1) * 4, hipMemcpyDeviceToDevice, stream_));
         HIPCHK(hipMemcpyAsync(col_.p, dCol, (size_t)nnz_ * 4, hipMemcpyDeviceToDevice, stream_));
     } else {
@@ -1032,57 +1118,8 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
     depth_ = hcnt[C_COUNT] + 1;
     tm.mark("split, transpose map, levels, sort");
 
-    // Orders: rows in order of groups of q consecutive levels, every group
-    // padded to a multiple of 64 rows so that a wavefront never holds rows of
-    // two groups, the whole padded to a multiple of BS; gate rows: for each
-    // 64-row segment of group G, one row of group G-dist (forward) and one of
-    // group G+dist (backward), spread over that group. Every level 0..depth-1
-    // holds at least one row, so every group is non-empty. The group layout
-    // follows from the first sorted row of each level (lvlStart, depth+1
-    // entries): computed on the host from that, rows scattered on the device.
-    std::vector<int> lvlStart(depth_ + 1);
-    struct Layout {
-        int ng = 0, P = 0;
-        std::vector<int> gStart, gFirst, gRows, gF, gB;
-    };
-    auto layout = [&](int q, int dist, bool gates, Layout& o) {
-        o.ng = (depth_ + q - 1) / q;
-        o.gStart.assign(o.ng, 0);
-        o.gFirst.assign(o.ng, 0);
-        o.gRows.assign(o.ng, 0);
-        long long pos = 0;
-        for (int G = 0; G < o.ng; ++G) {
-            const int first = lvlStart[G * q], end = lvlStart[std::min((G + 1) * q, depth_)];
-            o.gFirst[G] = first;
-            o.gRows[G] = end - first;
-            o.gStart[G] = (int)pos;
-            pos = (pos + o.gRows[G] + 63) / 64 * 64;
-        }
-        pos = (pos + BS - 1) / BS * BS;
-        o.P = (int)pos;
-        if (!gates) return;
-        const int nseg = o.P / 64;
-        o.gF.assign(nseg, -1);
-        o.gB.assign(nseg, -1);
-        std::vector<int> segG(nseg, -1);
-        for (int G = 0; G < o.ng; ++G) {
-            const int s0 = o.gStart[G] / 64, s1 = (o.gStart[G] + o.gRows[G] + 63) / 64;
-            for (int sg = s0; sg < s1; ++sg) segG[sg] = G;
-        }
-        for (int sg = 0; sg < nseg; ++sg) {
-            const int G = segG[sg];
-            if (G < 0) continue;
-            const unsigned h = (unsigned)sg * 2654435761u;
-            const int gf = G - dist, gb = G + dist;
-            if (gf >= 0) o.gF[sg] = o.gStart[gf] + (int)(h % (unsigned)o.gRows[gf]);
-            if (gb < o.ng) o.gB[sg] = o.gStart[gb] + (int)(h % (unsigned)o.gRows[gb]);
-        }
-    };
-    auto upload = [&](DevBuf& d, const void* src, size_t bytes) -> hipError_t {
-        hipError_t e = d.alloc(bytes);
-        if (e != hipSuccess) return e;
-        return hipMemcpyAsync(d.p, src, bytes, hipMemcpyHostToDevice, stream_);
-    };
+    std::vector<int>& lvlStart = hlvlStart_;
+    lvlStart.resize((size_t)depth_ + 1);
     HIPCHK(lvlStart_.alloc(((size_t)depth_ + 1) * 4));
     k_fill_i32<<<blocks(depth_ + 1), BS, 0, stream_>>>(lvlStart_.as<int>(), -1, depth_ + 1);
     k_level_starts<<<blocks(n), BS, 0, stream_>>>(n, sortKeys_.as<int>(), lvlStart_.as<int>());
@@ -1096,145 +1133,160 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
         err = "dependency levels are not contiguous";
         return ASTG_ERR_HIP;
     }
-    // the host-planner path (ASTG_HOST_PLAN) also needs the sorted rows and
-    // both orders on the host
-    std::vector<int> sortedLev, sortedRow, spadded;
-    if (hostPlan_) {
-        sortedLev.resize(n);
-        sortedRow.resize(n);
-        HIPCHK(hipMemcpyAsync(sortedLev.data(), sortKeys_.p, n4, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipMemcpyAsync(sortedRow.data(), sortRows_.p, n4, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-    }
-    // The host vectors uploaded below live until the synchronisation at the
-    // end of this function.
-    auto scatter = [&](const Layout& o, int q, DevBuf& ord) -> int {
-        HIPCHK(upload(grpStart_, o.gStart.data(), (size_t)o.ng * 4));
-        HIPCHK(upload(grpFirst_, o.gFirst.data(), (size_t)o.ng * 4));
-        HIPCHK(ord.alloc((size_t)o.P * 4));
-        k_fill_i32<<<blocks(o.P), BS, 0, stream_>>>(ord.as<int>(), -1, o.P);
-        k_pad_order<<<blocks(n), BS, 0, stream_>>>(n, sortKeys_.as<int>(), sortRows_.as<int>(), q,
-                                                  grpStart_.as<int>(), grpFirst_.as<int>(), ord.as<int>());
-        HIPCHK(hipGetLastError());
-        // the small group arrays are reused by the next call: finish this one
-        HIPCHK(hipStreamSynchronize(stream_));
-        return ASTG_OK;
-    };
     // factorisation: rows in level order, one launch per level
-    Layout lf, ls;
-    layout(1, 1, false, lf);
+    const LevelLayout lf = levelLayout(lvlStart, 1, 1, false);
     P_ = lf.P;
-    if (int rc = scatter(lf, 1, order_)) return rc;
+    if (int rc = scatterLevels(lf, 1, order_, err)) return rc;
     levRange_.assign(2 * (size_t)depth_, 0);
     for (int L = 0; L < depth_; ++L) {
         levRange_[2 * L] = lf.gStart[L];
         levRange_[2 * L + 1] = lf.gStart[L] + lf.gRows[L];
     }
     // PCG work vectors: sweep-ordered (PS entries) unless the row order is kept
-    const char* keep = getenv("ASTG_ROW_ORDER");
-    const bool keepRows = keep && atoi(keep) != 0;
-    perm_ = !rowOrderForced_ && !keepRows;
-    // sweeps: in tiles where they fit; otherwise q levels per group
-    if (!keepRows && !noTile_)
-        if (int rc = tileSetup(tiled_, err)) return rc;
-    if (!tiled_) {
-        layout(merge_, gateDist_, true, ls);
-        PS_ = ls.P;
-        if (int rc = scatter(ls, merge_, sorder_)) return rc;
-        HIPCHK(upload(sgateF_, ls.gF.data(), ls.gF.size() * 4));
-        HIPCHK(upload(sgateB_, ls.gB.data(), ls.gB.size() * 4));
-    }
-    if (hostPlan_) {
-        // the host construction of both orders and the gates, from the sorted
-        // rows, must give the device's entry for entry
-        std::vector<int> padded, gF, gB, devOrd, devF, devB;
-        hostOrder(1, 1, n, depth_, sortedLev, sortedRow, padded, gF, gB);
-        devOrd.resize(P_);
-        HIPCHK(hipMemcpyAsync(devOrd.data(), order_.p, (size_t)P_ * 4, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-        if ((int)padded.size() != P_ || padded != devOrd) {
-            err = "device-built factorisation order differs from the host construction";
-            return ASTG_ERR_HIP;
-        }
-        if (!tiled_) {
-            hostOrder(merge_, gateDist_, n, depth_, sortedLev, sortedRow, spadded, gF, gB);
-            devOrd.resize(PS_);
-            devF.resize(ls.gF.size());
-            devB.resize(ls.gB.size());
-            HIPCHK(hipMemcpyAsync(devOrd.data(), sorder_.p, (size_t)PS_ * 4, hipMemcpyDeviceToHost, stream_));
-            HIPCHK(hipStreamSynchronize(stream_));
-            if ((int)spadded.size() != PS_ || spadded != devOrd || gF != ls.gF || gB != ls.gB) {
-                err = "device-built sweep order or gates differ from the host construction";
-                return ASTG_ERR_HIP;
-            }
-        }
-    }
-    tm.mark("level and sweep orders");
-    // symbolic plans: factorisation programs and merged stencils
-    const int maxY = kMaxDeps;
+    keepRows_ = false;
+    if (const char* g = getenv("ASTG_ROW_ORDER")) keepRows_ = atoi(g) != 0;
+    tilesAsked_ = -1;
+    if (const char* g = getenv("ASTG_TILES")) tilesAsked_ = std::max(0, atoi(g));
+    perm_ = !rowOrderForced_ && !keepRows_;
+    tm.mark("level order");
+    // symbolic plan of the factorisation
     if (!hostPlan_) {
-        const int rc = planDevice(maxY, !tiled_, err);
-        if (rc) return rc;
+        if (int rc = planMicDevice(err)) return rc;
     } else {
-        std::vector<int> lend, ubeg;
+        // with ASTG_HOST_PLAN the host planners serve, and the host
+        // construction of every order must give the device's entry for entry
+        std::vector<int> padded, lend, ubeg;
+        if (int rc = checkOrder(lf, 1, 1, false, order_, padded, "factorisation order", err)) return rc;
         if (int rc = ensureHostPattern(err)) return rc;
-        const int* rowstart = hrs_.data();
-        const int* col = hcol_.data();
-        if (splitPatternHost(n, rowstart, col, lend, ubeg, err)) return ASTG_ERR_ARG;
+        if (splitPatternHost(n, hrs_.data(), hcol_.data(), lend, ubeg, err)) return ASTG_ERR_ARG;
         std::vector<long long> ms;
         std::vector<int> mp;
-        planMic(n, rowstart, lend.data(), ubeg.data(), col, ms, mp);
+        planMic(n, hrs_.data(), lend.data(), ubeg.data(), hcol_.data(), ms, mp);
         HIPCHK(upload(micStart_, ms.data(), ms.size() * 8));
         HIPCHK(upload(micProg_, mp.data(), mp.size() * 4));
         HIPCHK(hipStreamSynchronize(stream_));
-        std::vector<int> lev(n), pos(n);
-        for (int q = 0; q < n; ++q) lev[sortedRow[q]] = sortedLev[q];
-        for (int q = 0; q < PS_ && !tiled_; ++q)
-            if (spadded[q] >= 0) pos[spadded[q]] = q;
-        DevStencil* dst[2] = {&stF_, &stB_};
-        for (int dir = 0; dir < 2 && !tiled_; ++dir) {
-            SweepStencil st;
-            planStencil(dir, n, rowstart, lend.data(), ubeg.data(), col, lev.data(), merge_, maxY, spadded.data(),
-                        PS_, pos.data(), st);
-            DevStencil& D = *dst[dir];
-            D.E = (long long)st.idx.size();
-            HIPCHK(upload(D.start, st.start.data(), st.start.size() * 4));
-            HIPCHK(upload(D.nr, st.nr.data(), st.nr.size() * 4));
-            HIPCHK(upload(D.idx, st.idx.data(), st.idx.size() * 4));
-            HIPCHK(upload(D.ustart, st.ustart.data(), st.ustart.size() * 4));
-            HIPCHK(upload(D.upd, st.upd.data(), st.upd.size()));
-            HIPCHK(D.coef.alloc((size_t)D.E * 8));
-            // the host vectors must outlive the copies
-            HIPCHK(hipStreamSynchronize(stream_));
-        }
     }
     HIPCHK(live_.alloc((size_t)n));
-    if (perm_) {
-        const int rc = permuteSetup(err);
-        if (rc) return rc;
+    tm.mark("factorisation plan");
+    HIPCHK(hipStreamSynchronize(stream_));
+    patternSet_ = true;
+    return ASTG_OK;
+}
+
+// Merged sweeps (sweep_merge.h) of the current form: order, gates, stencils.
+int PcgDevice::mergedSetup(std::string& err) {
+    const LevelLayout ls = levelLayout(hlvlStart_, merge_, gateDist_, true);
+    f_->PS = ls.P;
+    if (int rc = scatterLevels(ls, merge_, f_->sorder, err)) return rc;
+    HIPCHK(upload(f_->sgateF, ls.gF.data(), ls.gF.size() * 4));
+    HIPCHK(upload(f_->sgateB, ls.gB.data(), ls.gB.size() * 4));
+    const int maxY = kMaxDeps;
+    if (!hostPlan_) {
+        if (int rc = planStencilsDevice(maxY, err)) return rc;
+        HIPCHK(hipStreamSynchronize(stream_));  // ls
+        return ASTG_OK;
     }
+    const int n = n_;
+    std::vector<int> spadded, lend, ubeg;
+    if (int rc = checkOrder(ls, merge_, gateDist_, true, f_->sorder, spadded, "sweep order or gates", err)) return rc;
+    if (int rc = ensureHostPattern(err)) return rc;
+    if (splitPatternHost(n, hrs_.data(), hcol_.data(), lend, ubeg, err)) return ASTG_ERR_ARG;
+    std::vector<int> lev(n), pos(n);
+    HIPCHK(hipMemcpyAsync(lev.data(), lev_.p, (size_t)n * 4, hipMemcpyDeviceToHost, stream_));
+    HIPCHK(hipStreamSynchronize(stream_));
+    for (int q = 0; q < f_->PS; ++q)
+        if (spadded[q] >= 0) pos[spadded[q]] = q;
+    DevStencil* dst[2] = {&f_->stF, &f_->stB};
+    for (int dir = 0; dir < 2; ++dir) {
+        SweepStencil st;
+        planStencil(dir, n, hrs_.data(), lend.data(), ubeg.data(), hcol_.data(), lev.data(), merge_, maxY,
+                    spadded.data(), f_->PS, pos.data(), st);
+        DevStencil& D = *dst[dir];
+        D.E = (long long)st.idx.size();
+        HIPCHK(upload(D.start, st.start.data(), st.start.size() * 4));
+        HIPCHK(upload(D.nr, st.nr.data(), st.nr.size() * 4));
+        HIPCHK(upload(D.idx, st.idx.data(), st.idx.size() * 4));
+        HIPCHK(upload(D.ustart, st.ustart.data(), st.ustart.size() * 4));
+        HIPCHK(upload(D.upd, st.upd.data(), st.upd.size()));
+        HIPCHK(D.coef.alloc((size_t)D.E * 8));
+        // the host vectors must outlive the copies
+        HIPCHK(hipStreamSynchronize(stream_));
+    }
+    return ASTG_OK;
+}
+
+// Builds the sweeps of the pattern into f, which becomes the current form: in
+// tiles of `width`-byte values where they are tried and serve, otherwise merged,
+// or not at all (f not ready).
+int PcgDevice::buildForm(SweepForm& f, int width, bool tryTiles, bool orMerged, std::string& err) {
+    PhaseTimer tm("sweeps");
+    f_ = &f;
+    f.tiled = f.coef64 = f.f32 = false;
+    if (tryTiles && !keepRows_)
+        if (int rc = tileSetup(width, f.tiled, err)) return rc;
+    tm.mark("tiles");
+    if (!f.tiled) {
+        if (!orMerged) return ASTG_OK;
+        if (int rc = mergedSetup(err)) return rc;
+        tm.mark("merged order and stencils");
+    }
+    if (perm_)
+        if (int rc = permuteSetup(err)) return rc;
+    // persistent grids (all blocks co-resident)
+    if (f.tiled) {
+        f.gF64 = f.gF32 = f.gB64 = f.gB32 = f.tileK;
+        if (K_)
+            if (int rc = tileSystems(err)) return rc;
+    } else {
+        const int schunks = f.PS / BS;
+        f.gF64 = coopBlocks(k_fwd<double>, cus_, schunks);
+        f.gF32 = coopBlocks(k_fwd<float>, cus_, schunks);
+        f.gB64 = coopBlocks(k_bwd_dot<double>, cus_, schunks);
+        f.gB32 = coopBlocks(k_bwd_dot<float>, cus_, schunks);
+    }
+    f.ready = true;
+    tm.mark("permuted pattern");
+    return ASTG_OK;
+}
+
+// Work vectors of the current form.
+int PcgDevice::formVectors(std::string& err) {
     const size_t nv8 = (size_t)vlen() * 8;
     HIPCHK(r_.alloc(nv8));
     HIPCHK(z_.alloc(nv8));
     HIPCHK(s_.alloc(nv8));
     HIPCHK(q_.alloc(nv8));
-    HIPCHK(y_.alloc((size_t)PS_ * (tiled_ ? 1 : 2) * 8));
-    if (!tiled_) HIPCHK(zp_.alloc((size_t)PS_ * 8));
-    tm.mark("symbolic plans");
-    // persistent grids (all blocks co-resident)
-    if (tiled_) {
-        gF64_ = gF32_ = gB64_ = gB32_ = tileK_;
-    } else {
-        const int schunks = PS_ / BS;
-        gF64_ = coopBlocks(k_fwd<double>, cus, schunks);
-        gF32_ = coopBlocks(k_fwd<float>, cus, schunks);
-        gB64_ = coopBlocks(k_bwd_dot<double>, cus, schunks);
-        gB32_ = coopBlocks(k_bwd_dot<float>, cus, schunks);
-    }
-    gb_ = std::max(std::max(gB64_, gB32_), 1);
+    HIPCHK(y_.alloc((size_t)f_->PS * (f_->tiled ? 1 : 2) * 8));
+    if (!f_->tiled) HIPCHK(zp_.alloc((size_t)f_->PS * 8));
+    gb_ = std::max({f_->gF64, f_->gF32, f_->gB64, f_->gB32, 1});
     HIPCHK(part_.alloc((size_t)(2 * gs_ + 2 * gb_ + 8) * 8));
-    HIPCHK(hipStreamSynchronize(stream_));
     return ASTG_OK;
+}
+
+// A mixed solve takes FP32-only tiles (form 1) where the pattern asks for them
+// and has them; every other solve takes form 0. Both stay once they are built:
+// a caller that alternates keeps the faster sweeps of each precision (one form
+// for both made every mixed solve after an FP64 one sweep merged, and a caller
+// with a new pattern per FP64 step build two).
+int PcgDevice::useForm(int precision, std::string& err) {
+    if (!patternSet_) {
+        err = "no solver pattern";
+        return ASTG_ERR_STATE;
+    }
+    if (precision != ASTG_PREC_FP64 && tileFp32_ && !narrowTried_ && !(form_[0].ready && form_[0].tiled)) {
+        if (int rc = buildForm(form_[1], 4, true, false, err)) return rc;
+        narrowTried_ = true;
+        if (form_[1].ready && !form_[0].ready && tilesFit(8)) std::swap(form_[0], form_[1]);  // they serve both
+    }
+    if (precision != ASTG_PREC_FP64 && form_[1].ready) {
+        f_ = &form_[1];
+        return formVectors(err);
+    }
+    // tiles that were tried in FP32, and do not exist or fit FP32 only, are not tried in FP64
+    if (!form_[0].ready)
+        if (int rc = buildForm(form_[0], 8, !narrowTried_, true, err)) return rc;
+    f_ = &form_[0];
+    return formVectors(err);
 }
 
 template <typename T>
@@ -1253,59 +1305,59 @@ void PcgDevice::launchSpmv(int n, const int* rs, const int* col, const T* A, con
 }
 
 int PcgDevice::permuteSetup(std::string& err) {
-    const int n = n_, P = PS_;
+    const int n = n_, P = f_->PS;
     const long long nnz = nnz_;
-    HIPCHK(pos_.alloc((size_t)n * 4));
-    HIPCHK(prs_.alloc(((size_t)P + 1) * 4));
-    HIPCHK(pcol_.alloc((size_t)nnz * 4));
-    HIPCHK(pmap_.alloc((size_t)nnz * 4));
-    HIPCHK(valP_.alloc((size_t)nnz * 8));
-    HIPCHK(invdP_.alloc((size_t)P * 8));
-    HIPCHK(bP_.alloc((size_t)P * 8));
-    HIPCHK(xP_.alloc((size_t)P * 8));
+    HIPCHK(f_->pos.alloc((size_t)n * 4));
+    HIPCHK(f_->prs.alloc(((size_t)P + 1) * 4));
+    HIPCHK(f_->pcol.alloc((size_t)nnz * 4));
+    HIPCHK(f_->pmap.alloc((size_t)nnz * 4));
+    HIPCHK(f_->valP.alloc((size_t)nnz * 8));
+    HIPCHK(f_->invdP.alloc((size_t)P * 8));
+    HIPCHK(f_->bP.alloc((size_t)P * 8));
+    HIPCHK(f_->xP.alloc((size_t)P * 8));
     HIPCHK(permLen_.alloc((size_t)P * 4));
-    const int* order = sorder_.as<int>();
-    if (!tiled_) {
-        k_row_pos<<<blocks(P), BS, 0, stream_>>>(P, order, pos_.as<int>());
-        k_rterm_pos<<<blocks(P), BS, 0, stream_>>>(P, stF_.start.as<int>(), stF_.nr.as<int>(), stF_.idx.as<int>(),
-                                                   pos_.as<int>());
+    const int* order = f_->sorder.as<int>();
+    if (!f_->tiled) {
+        k_row_pos<<<blocks(P), BS, 0, stream_>>>(P, order, f_->pos.as<int>());
+        k_rterm_pos<<<blocks(P), BS, 0, stream_>>>(P, f_->stF.start.as<int>(), f_->stF.nr.as<int>(), f_->stF.idx.as<int>(),
+                                                   f_->pos.as<int>());
     }
     k_perm_len<<<blocks(P), BS, 0, stream_>>>(P, order, rs_.as<int>(), permLen_.as<int>());
     size_t tb = 0;
-    HIPCHK(hipcub::DeviceScan::InclusiveSum(nullptr, tb, permLen_.as<int>(), prs_.as<int>() + 1, P, stream_));
+    HIPCHK(hipcub::DeviceScan::InclusiveSum(nullptr, tb, permLen_.as<int>(), f_->prs.as<int>() + 1, P, stream_));
     HIPCHK(planTmp_.alloc(tb));
-    HIPCHK(hipcub::DeviceScan::InclusiveSum(planTmp_.p, tb, permLen_.as<int>(), prs_.as<int>() + 1, P, stream_));
-    k_fill_i32<<<1, BS, 0, stream_>>>(prs_.as<int>(), 0, 1);
-    k_perm_fill<<<blocks(P), BS, 0, stream_>>>(P, order, rs_.as<int>(), col_.as<int>(), pos_.as<int>(),
-                                               prs_.as<int>(), pcol_.as<int>(), pmap_.as<int>());
+    HIPCHK(hipcub::DeviceScan::InclusiveSum(planTmp_.p, tb, permLen_.as<int>(), f_->prs.as<int>() + 1, P, stream_));
+    k_fill_i32<<<1, BS, 0, stream_>>>(f_->prs.as<int>(), 0, 1);
+    k_perm_fill<<<blocks(P), BS, 0, stream_>>>(P, order, rs_.as<int>(), col_.as<int>(), f_->pos.as<int>(),
+                                               f_->prs.as<int>(), f_->pcol.as<int>(), f_->pmap.as<int>());
     HIPCHK(hipGetLastError());
     return ASTG_OK;
 }
 
 int PcgDevice::prepareSolve(std::string& err) {
     if (!perm_) return ASTG_OK;
-    const int P = PS_;
-    const int* order = sorder_.as<int>();
+    const int P = f_->PS;
+    const int* order = f_->sorder.as<int>();
     k_gather_vals<<<std::max(1, std::min(8 * cus_, blocks(nnz_))), BS, 0, stream_>>>(
-        (long)nnz_, pmap_.as<int>(), val_.as<double>(), valP_.as<double>());
-    k_to_sweep<<<blocks(P), BS, 0, stream_>>>(P, order, invd_.as<double>(), invdP_.as<double>());
-    k_to_sweep<<<blocks(P), BS, 0, stream_>>>(P, order, b_.as<double>(), bP_.as<double>());
+        (long)nnz_, f_->pmap.as<int>(), val_.as<double>(), f_->valP.as<double>());
+    k_to_sweep<<<blocks(P), BS, 0, stream_>>>(P, order, invd_.as<double>(), f_->invdP.as<double>());
+    k_to_sweep<<<blocks(P), BS, 0, stream_>>>(P, order, b_.as<double>(), f_->bP.as<double>());
     HIPCHK(hipGetLastError());
     return ASTG_OK;
 }
 
 bool PcgDevice::isSweepKernel(const void* f) const {
-    return isTileKernel(f) || f == (const void*)k_fwd<double> || f == (const void*)k_fwd<float> || f == (const void*)k_bwd_dot<double> ||
-           f == (const void*)k_bwd_dot<float>;
+    return isTileKernel(f) || f == (const void*)k_fwd<double> || f == (const void*)k_fwd<float> ||
+           f == (const void*)k_bwd_dot<double> || f == (const void*)k_bwd_dot<float>;
 }
 
 SweepPlan PcgDevice::splan() const {
     SweepPlan s;
-    s.order = sorder_.as<int>();
-    s.gateF = sgateF_.as<int>();
-    s.gateB = sgateB_.as<int>();
-    s.P = PS_;
-    s.nchunks = PS_ / BS;
+    s.order = f_->sorder.as<int>();
+    s.gateF = f_->sgateF.as<int>();
+    s.gateB = f_->sgateB.as<int>();
+    s.P = f_->PS;
+    s.nchunks = f_->PS / BS;
     s.pollCap = pollCap_;
     s.gateCap = gateCap_;
     s.trace = trace_;
@@ -1376,11 +1428,11 @@ int PcgDevice::launchMic(double tau, double ratio, std::string& err) {
 }
 
 int PcgDevice::launchMerge(std::string& err) {
-    const DevStencil* st[2] = {&stF_, &stB_};
+    const DevStencil* st[2] = {&f_->stF, &f_->stB};
     for (int dir = 0; dir < 2; ++dir) {
         const DevStencil& d = *st[dir];
         auto k = dir == 0 ? k_merge<0> : k_merge<1>;
-        k<<<blocks(PS_), BS, 0, stream_>>>(PS_, sorder_.as<int>(), rs_.as<int>(), lend_.as<int>(), ubeg_.as<int>(),
+        k<<<blocks(f_->PS), BS, 0, stream_>>>(f_->PS, f_->sorder.as<int>(), rs_.as<int>(), lend_.as<int>(), ubeg_.as<int>(),
                                            F_.as<double>(), invd_.as<double>(), d.start.as<int>(), d.nr.as<int>(),
                                            d.idx.as<int>(), d.ustart.as<int>(), d.upd.as<uint8_t>(),
                                            d.coef.as<double>(), perm_ ? 1 : 0);
@@ -1392,30 +1444,37 @@ int PcgDevice::launchMerge(std::string& err) {
 // FP32 copies of A, the pivots and the merged stencil coefficients.
 int PcgDevice::convert32(std::string& err) {
     const long long nnz = nnz_;
-    HIPCHK(val32_.alloc((size_t)nnz * 4));
-    HIPCHK(invd32_.alloc((size_t)vlen() * 4));
-    k_d2f<<<blocks(nnz), BS, 0, stream_>>>(sVal64(), val32_.as<float>(), nnz);
-    k_d2f<<<blocks(vlen()), BS, 0, stream_>>>(sInvd64(), invd32_.as<float>(), vlen());
-    if (tiled_) {
+    HIPCHK(f_->val32.alloc((size_t)nnz * 4));
+    HIPCHK(f_->invd32.alloc((size_t)vlen() * 4));
+    k_d2f<<<blocks(nnz), BS, 0, stream_>>>(sVal64(), f_->val32.as<float>(), nnz);
+    k_d2f<<<blocks(vlen()), BS, 0, stream_>>>(sInvd64(), f_->invd32.as<float>(), vlen());
+    if (f_->tiled) {
         if (int rc = tileCoef<float>(err)) return rc;
-        f32Valid_ = true;
+        f_->f32 = true;
         return ASTG_OK;
     }
-    HIPCHK(stF_.coef32.alloc((size_t)stF_.E * 4));
-    HIPCHK(stB_.coef32.alloc((size_t)stB_.E * 4));
-    k_d2f<<<blocks(stF_.E), BS, 0, stream_>>>(stF_.coef.as<double>(), stF_.coef32.as<float>(), stF_.E);
-    k_d2f<<<blocks(stB_.E), BS, 0, stream_>>>(stB_.coef.as<double>(), stB_.coef32.as<float>(), stB_.E);
+    if (int rc = ensureCoef64(err)) return rc;
+    HIPCHK(f_->stF.coef32.alloc((size_t)f_->stF.E * 4));
+    HIPCHK(f_->stB.coef32.alloc((size_t)f_->stB.E * 4));
+    k_d2f<<<blocks(f_->stF.E), BS, 0, stream_>>>(f_->stF.coef.as<double>(), f_->stF.coef32.as<float>(), f_->stF.E);
+    k_d2f<<<blocks(f_->stB.E), BS, 0, stream_>>>(f_->stB.coef.as<double>(), f_->stB.coef32.as<float>(), f_->stB.E);
     HIPCHK(hipGetLastError());
-    f32Valid_ = true;
+    f_->f32 = true;
     return ASTG_OK;
 }
 
 int PcgDevice::factor(double tau, double ratio, std::string& err) {
-    f32Valid_ = false;  // new values and pivots: the FP32 copies are stale
-    int rc = launchMic(tau, ratio, err);
-    if (rc) return rc;
-    tileCoef64_ = false;  // tile coefficients are gathered by the solve, in its precision
-    return tiled_ ? ASTG_OK : launchMerge(err);
+    // the sweeps' coefficients are formed by the solve, in its form and precision
+    for (SweepForm& f : form_) f.coef64 = f.f32 = false;
+    return launchMic(tau, ratio, err);
+}
+
+// FP64 coefficients of the current form's sweeps, once per factor.
+int PcgDevice::ensureCoef64(std::string& err) {
+    if (f_->coef64) return ASTG_OK;
+    if (int rc = f_->tiled ? tileCoef<double>(err) : launchMerge(err)) return rc;
+    f_->coef64 = true;
+    return ASTG_OK;
 }
 
 int PcgDevice::syncScalars(std::string& err) {
@@ -1428,7 +1487,7 @@ template <typename T>
 int PcgDevice::launchFwd(const T* invd, const T* r, int k, int mode, int it, int maxIt, int norm, double tolRel,
                          std::string& err) {
     const int g = fwdGrid<T>(), gb = bwdGrid<T>();
-    const StencilView<T> V = view<T>(stF_);
+    const StencilView<T> V = view<T>(f_->stF);
     T* y = ybuf<T>(k);
     HIPCHK(launchCoop(coop_, k_fwd<T>, g, stream_, splan(), V, invd, r, y, zp_.as<T>(), parts(gb), cnt_.as<int>(),
                       scal_.as<double>(), mode, it, maxIt, norm, tolRel));
@@ -1438,7 +1497,7 @@ int PcgDevice::launchFwd(const T* invd, const T* r, int k, int mode, int it, int
 template <typename T>
 int PcgDevice::launchBwd(const T* invd, const T* r, T* z, int k, int parityOut, std::string& err) {
     const int gb = bwdGrid<T>();
-    const StencilView<T> V = view<T>(stB_);
+    const StencilView<T> V = view<T>(f_->stB);
     const T* y = ybuf<T>(k);
     T* ynext = ybuf<T>(k + 1);
     HIPCHK(launchCoop(coop_, k_bwd_dot<T>, gb, stream_, splan(), V, invd, y, ynext, r, z, zp_.as<T>(), parts(gb),
@@ -1446,31 +1505,21 @@ int PcgDevice::launchBwd(const T* invd, const T* r, T* z, int k, int parityOut, 
     return ASTG_OK;
 }
 
-// A pattern whose tiles fit the LDS in FP32 only, asked for an FP64 solve: the
-// merged sweeps from here on (the values and the factor stay).
-int PcgDevice::dropTiles(std::string& err) {
-    PhaseTimer tm("setPattern (merged sweeps)");
-    noTile_ = true;
-    const int rc = setPatternImpl(n_, nnz_, rs_.as<int>(), col_.as<int>(), tm, err);
-    noTile_ = false;
-    return rc ? rc : launchMerge(err);
-}
-
 // The values that the first sweep of a solve waits for.
 template <typename T>
 void PcgDevice::armSweeps() {
-    if (!tiled_) {
-        k_fill_sent<T><<<blocks(2 * PS_), BS, 0, stream_>>>(y_.as<T>(), 2 * PS_);
+    if (!f_->tiled) {
+        k_fill_sent<T><<<blocks(2 * f_->PS), BS, 0, stream_>>>(y_.as<T>(), 2 * f_->PS);
         return;
     }
     for (int d = 0; d < 2; ++d)
-        if (const int h = 2 * tile_[d].halo) k_fill_sent<T><<<blocks(h), BS, 0, stream_>>>(tile_[d].inbox.as<T>(), h);
+        if (const int h = 2 * f_->tile[d].halo) k_fill_sent<T><<<blocks(h), BS, 0, stream_>>>(f_->tile[d].inbox.as<T>(), h);
 }
 
 template <typename T>
 int PcgDevice::precondition(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm,
                             double tolRel, std::string& err) {
-    if (tiled_) return launchTile<T>(invd, r, z, k, mode, it, maxIt, norm, tolRel, 3, err);
+    if (f_->tiled) return launchTile<T>(invd, r, z, k, mode, it, maxIt, norm, tolRel, 3, err);
     if (int rc = launchFwd<T>(invd, r, k, mode, it, maxIt, norm, tolRel, err)) return rc;
     return launchBwd<T>(invd, r, z, k, k & 1, err);
 }
@@ -1504,7 +1553,7 @@ int PcgDevice::pcgInner(const T* A, const T* invd, const T* b, double* x, double
     if (rc) return rc;
     // z as the PCG reads it: with merged sweeps in sweep order the backward
     // sweep's published copy (valid until the next forward sweep re-arms it)
-    const T* zv = perm_ && !tiled_ ? zp_.as<T>() : z;
+    const T* zv = perm_ && !f_->tiled ? zp_.as<T>() : z;
     k_xpby<T><<<gs, BS, 0, stream_>>>(n, zv, s, Pt, scal, 0, 0);
     HIPCHK(hipGetLastError());
     int it = 0;
@@ -1551,13 +1600,9 @@ int PcgDevice::solve(const astg_pcg_params& prm, astg_pcg_result& res, std::stri
 }
 
 int PcgDevice::solveOnce(const astg_pcg_params& prm, astg_pcg_result& res, std::string& err) {
-    if (tiled_ && prm.precision == ASTG_PREC_FP64) {
-        if (!tilesFit(tileSlots_, 8)) {
-            if (int rc = dropTiles(err)) return rc;
-        } else if (int rc = ensureTileCoef64(err)) {
-            return rc;
-        }
-    }
+    if (int rc = useForm(prm.precision, err)) return rc;
+    if (prm.precision == ASTG_PREC_FP64)
+        if (int rc = ensureCoef64(err)) return rc;
     const int n = vlen(), gs = gs_;
     res.n = n_;
     res.nnz = nnz_;
@@ -1566,7 +1611,7 @@ int PcgDevice::solveOnce(const astg_pcg_params& prm, astg_pcg_result& res, std::
     if (int rc = prepareSolve(err)) return rc;
     // the solution in row order (x_) from the sweep-ordered one
     auto finish = [&]() -> int {
-        if (perm_) k_from_sweep<<<blocks(PS_), BS, 0, stream_>>>(PS_, sorder_.as<int>(), sX(), x_.as<double>());
+        if (perm_) k_from_sweep<<<blocks(f_->PS), BS, 0, stream_>>>(f_->PS, f_->sorder.as<int>(), sX(), x_.as<double>());
         HIPCHK(hipGetLastError());
         return ASTG_OK;
     };
@@ -1602,7 +1647,7 @@ int PcgDevice::solveOnce(const astg_pcg_params& prm, astg_pcg_result& res, std::
     double rnorm = 0;
     bool conv = false;
     for (;;) {
-        const Parts Pt = parts(gB64_);
+        const Parts Pt = parts(f_->gB64);
         k_residual64<<<gs, BS, 0, stream_>>>(n, sRs(), sCol(), sVal64(), sX(), sB(), r64_.as<double>(), Pt,
                                              prm.norm);
         k_res_final<<<1, BS, 0, stream_>>>(Pt, scal_.as<double>(), prm.norm);
@@ -1632,7 +1677,7 @@ int PcgDevice::solveOnce(const astg_pcg_params& prm, astg_pcg_result& res, std::
         int it = 0;
         double ir = 0;
         bool ic = false;
-        rc = pcgInner<float>(val32_.as<float>(), invd32_.as<float>(), rhs32, d64, eta, prm.max_iterations - total,
+        rc = pcgInner<float>(f_->val32.as<float>(), f_->invd32.as<float>(), rhs32, d64, eta, prm.max_iterations - total,
                              prm.norm, it, ir, ic, err, rhs64, mixedReplace_);
         if (rc) return rc;
         total += it;
@@ -1679,37 +1724,38 @@ int PcgDevice::downloadFactor(std::vector<double>& invdiag, std::vector<unsigned
 }
 
 int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, std::string& err) {
-    const int n = n_, nv = vlen();
+    const int n = n_;
     const long long nnz = nnz_, nl = nnzL();
+    const bool f32 = which == ASTG_K_SPMV32 || which == ASTG_K_FWD32 || which == ASTG_K_BWD32;
+    const bool sweep64s = which == ASTG_K_FWD64 || which == ASTG_K_BWD64;
+    // the form that a solve of the kernel's precision takes; the others run in the current one
+    if (f32 || sweep64s || !f_->ready) {
+        if (int rc = useForm(f32 ? ASTG_PREC_MIXED : ASTG_PREC_FP64, err)) return rc;
+    }
+    const int nv = vlen();
     // the solve's own layout: sweep-ordered vectors and CSR unless the row order is kept
     if (int rc = prepareSolve(err)) return rc;
     const int* rs = sRs();
     const int* col = sCol();
     double* scal = scal_.as<double>();
-    const bool f32 = which == ASTG_K_SPMV32 || which == ASTG_K_FWD32 || which == ASTG_K_BWD32;
-    if (f32 && !f32Valid_) {
+    if (f32 && !f_->f32) {
         int rc = convert32(err);
         if (rc) return rc;
     }
-    if (tiled_ && (which == ASTG_K_FWD64 || which == ASTG_K_BWD64)) {
-        if (!tilesFit(tileSlots_, 8)) {
-            err = "the FP64 sweeps of this ordering need a FP64 solve first";
-            return ASTG_ERR_STATE;
-        }
-        if (int rc = ensureTileCoef64(err)) return rc;
-    }
+    if (sweep64s)
+        if (int rc = ensureCoef64(err)) return rc;
     // one direction of a sweep
     auto sweep64 = [&](int dir) -> int {
         const double* iv = sInvd64();
-        if (tiled_)
+        if (f_->tiled)
             return launchTile<double>(iv, r_.as<double>(), z_.as<double>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30,
                                       1 << dir, err);
         return dir == 0 ? launchFwd<double>(iv, r_.as<double>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30, err)
                         : launchBwd<double>(iv, r_.as<double>(), z_.as<double>(), 0, 0, err);
     };
     auto sweep32 = [&](int dir) -> int {
-        const float* iv = invd32_.as<float>();
-        if (tiled_)
+        const float* iv = f_->invd32.as<float>();
+        if (f_->tiled)
             return launchTile<float>(iv, r_.as<float>(), z_.as<float>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30,
                                      1 << dir, err);
         return dir == 0 ? launchFwd<float>(iv, r_.as<float>(), 0, 0, 0, 1 << 30, ASTG_NORM_INF, 1e-30, err)
@@ -1722,23 +1768,23 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
             bytes = (w + 4) * nnz + 4.0 * (n + 1) + 3 * w * n;
             break;
         case ASTG_K_FWD64: case ASTG_K_FWD32: case ASTG_K_BWD64: case ASTG_K_BWD32:
-            if (tiled_) {
+            if (f_->tiled) {
                 // coefficients + slots of the stored entries; per position: r or y, pivot, y or z
                 // written, gate, flag (backward also r for the dot); per halo entry: source, value
                 const bool bw = which == ASTG_K_BWD64 || which == ASTG_K_BWD32;
-                bytes = (w + 2) * tile_[bw ? 1 : 0].E + ((bw ? 4.0 : 3.0) * w + 3) * PS_;
+                bytes = (w + 2) * f_->tile[bw ? 1 : 0].E + ((bw ? 4.0 : 3.0) * w + 3) * f_->PS;
                 break;
             }
             if (which == ASTG_K_BWD64 || which == ASTG_K_BWD32) {
                 // stencil coefficients + indices; per row: order, start, r-term count, y, next y
                 // armed, pivot, r, z published (and, in row order, written to the PCG vector),
                 // z gathered once
-                bytes = (w + 4) * stB_.E + ((perm_ ? 6.0 : 7.0) * w + 12) * n;
+                bytes = (w + 4) * f_->stB.E + ((perm_ ? 6.0 : 7.0) * w + 12) * n;
                 break;
             }
             // stencil coefficients + indices; per row: order, start, r-term count, r, pivot,
             // y written, y gathered once, backward vector armed
-            bytes = (w + 4) * stF_.E + (5.0 * w + 12) * n;
+            bytes = (w + 4) * f_->stF.E + (5.0 * w + 12) * n;
             break;
         case ASTG_K_MIC:
             // A values + pattern read, factor written twice (both triangles), invd
@@ -1765,10 +1811,10 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
         const Parts P64 = parts(bwdGrid<double>()), P32 = parts(bwdGrid<float>());
         if (sweep && f32) {
             armSweeps<float>();
-            if (!tiled_) k_fill_sent<float><<<blocks(PS_), BS, 0, stream_>>>(zp_.as<float>(), PS_);
+            if (!f_->tiled) k_fill_sent<float><<<blocks(f_->PS), BS, 0, stream_>>>(zp_.as<float>(), f_->PS);
         } else if (sweep) {
             armSweeps<double>();
-            if (!tiled_) k_fill_sent<double><<<blocks(PS_), BS, 0, stream_>>>(zp_.as<double>(), PS_);
+            if (!f_->tiled) k_fill_sent<double><<<blocks(f_->PS), BS, 0, stream_>>>(zp_.as<double>(), f_->PS);
         }
         // the forward sweep starts in mode 0, which needs nonzero ||b|| partials
         if (sweep) k_fill64<<<blocks(gs_), BS, 0, stream_>>>(gs_, P64.res, 1.0);
@@ -1784,7 +1830,7 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
                                                            q_.as<double>(), P64, scal);
                 break;
             case ASTG_K_SPMV32:
-                launchSpmv<float>(nv, rs, col, val32_.as<float>(), s_.as<float>(),
+                launchSpmv<float>(nv, rs, col, f_->val32.as<float>(), s_.as<float>(),
                                                           q_.as<float>(), P32, scal);
                 break;
             case ASTG_K_FWD64:

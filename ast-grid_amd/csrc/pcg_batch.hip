@@ -300,7 +300,10 @@ int PcgDevice::setBatch(const std::vector<int>& segRow, std::string& err) {
     HIPCHK(hipMemcpyAsync(segChunk_.p, segChunk.data(), (size_t)(K + 1) * 4, hipMemcpyHostToDevice, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
     K_ = K;
-    return tiled_ ? tileSystems(err) : ASTG_OK;
+    // the sweeps of this pattern are set up by its first solve, after this
+    if (!form_[0].ready || !form_[0].tiled) return ASTG_OK;
+    f_ = &form_[0];
+    return tileSystems(err);
 }
 
 int PcgDevice::batchGrid() const {
@@ -502,6 +505,7 @@ int PcgDevice::solveBatchOnce(const astg_pcg_params& prm, std::vector<astg_pcg_r
         err = "no batch layout";
         return ASTG_ERR_ARG;
     }
+    if (int rc = useForm(prm.precision, err)) return rc;
     const BatchView V = bview();
     const int g = batchGrid();
     const int maxIt = std::max(0, prm.max_iterations);
@@ -513,7 +517,7 @@ int PcgDevice::solveBatchOnce(const astg_pcg_params& prm, std::vector<astg_pcg_r
     std::vector<double> st((size_t)K * B_COUNT, 0.0);
     auto S = [&](int k, int slot) -> double& { return st[(size_t)k * B_COUNT + slot]; };
     if (prm.precision == ASTG_PREC_FP64) {
-        if (int rc = ensureTileCoef64(err)) return rc;
+        if (int rc = ensureCoef64(err)) return rc;
         for (int k = 0; k < K; ++k) {
             S(k, B_TOLREL) = prm.tol;
             S(k, B_MAXIT) = maxIt;
@@ -606,7 +610,7 @@ int PcgDevice::solveBatchOnce(const astg_pcg_params& prm, std::vector<astg_pcg_r
         if (!active) break;
         if ((rc = batchState(st, true, err))) return rc;
         kb_scale_rhs<<<g, BS, 0, stream_>>>(V, r64_.as<double>(), rhs64, rhs32);
-        rc = pcgBatchInner<float>(val32_.as<float>(), invd32_.as<float>(), rhs32, d64, innerMax, prm.norm, err, rhs64,
+        rc = pcgBatchInner<float>(f_->val32.as<float>(), f_->invd32.as<float>(), rhs32, d64, innerMax, prm.norm, err, rhs64,
                                   mixedReplace_);
         if (rc) return rc;
         kb_add_corr<<<g, BS, 0, stream_>>>(V, x_.as<double>(), d64);

@@ -643,10 +643,8 @@ void tileGrid(int K, const int* ext, int* k) {
 
 }  // namespace
 
-bool PcgDevice::tilesFit(int slots, int width) const {
-    return tileLds(slots, width) <= kTileLdsBytes;
-}
-size_t PcgDevice::tileLds(int slots, int width) const { return (size_t)slots * width + (size_t)tileExports_ * 6; }
+bool PcgDevice::tilesFit(int width) const { return tileLds(width) <= kTileLdsBytes; }
+size_t PcgDevice::tileLds(int width) const { return (size_t)f_->tileSlots * width + (size_t)f_->tileExports * 6; }
 
 // The system of every position of the batched form's tiles (0 at padding).
 static __global__ void k_tile_sys(int P, const int* order, const int* chunkSeg, int* sys) {
@@ -654,8 +652,8 @@ static __global__ void k_tile_sys(int P, const int* order, const int* chunkSeg, 
     if (t < P) sys[t] = order[t] >= 0 ? chunkSeg[order[t] / BS] : 0;
 }
 int PcgDevice::tileSystems(std::string& err) {
-    HIPCHK(tileSys_.alloc((size_t)PS_ * 4));
-    k_tile_sys<<<blocks(PS_), BS, 0, stream_>>>(PS_, sorder_.as<int>(), chunkSeg_.as<int>(), tileSys_.as<int>());
+    HIPCHK(f_->tileSys.alloc((size_t)f_->PS * 4));
+    k_tile_sys<<<blocks(f_->PS), BS, 0, stream_>>>(f_->PS, f_->sorder.as<int>(), chunkSeg_.as<int>(), f_->tileSys.as<int>());
     HIPCHK(hipGetLastError());
     return ASTG_OK;
 }
@@ -668,26 +666,22 @@ bool PcgDevice::mayTile(long long n, int width) {
     return (n + cus - 1) / std::max(1, cus) * width <= (long long)kTileLdsBytes;
 }
 
-int PcgDevice::tileSetup(bool& used, std::string& err) {
+int PcgDevice::tileSetup(int width, bool& used, std::string& err) {
     used = false;
     const int n = n_;
-    const bool placed = coordExt_[0] > 0;
+    const bool placed = coordExt_[0] > 0 && coordN_ == n;
     // a batch's chains end at its systems' boundaries, so its ranges are half as long
     // (6 systems of 12^3 to 56^3, FP32, ms per solve: 12 tiles 10.7, 16 9.7, 24 9.2, 48 9.6)
     const int range = rowOrderForced_ ? kTileRangeRows / 2 : kTileRangeRows;
     int K = std::min(cus_, placed ? std::max(1, n / kTileRows) : (n + range - 1) / range);
-    const char* forced = getenv("ASTG_TILES");
-    if (forced) {
-        if (atoi(forced) <= 0) return ASTG_OK;
-        K = std::min(atoi(forced), cus_);
-    }
+    if (tilesAsked_ == 0) return ASTG_OK;
+    if (tilesAsked_ > 0) K = std::min(tilesAsked_, cus_);
     int kk[3] = {1, 1, K};  // tiles per axis
     if (placed) {
         tileGrid(K, coordExt_, kk);
         K = kk[0] * kk[1] * kk[2];
     }
     if (K > n) return ASTG_OK;
-    const int width = tileFp32_ ? 4 : 8;  // of the values the tiles have to hold
     const long long S64 = (((long long)n + K - 1) / K + 63) / 64 * 64;
     // rows alone that do not fit: nothing is set up
     if (S64 >= 65535 || S64 * width > (long long)kTileLdsBytes || ((long long)K * depth_ << kWidthBits) >= (1ll << 32) ||
@@ -735,13 +729,13 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
     k_tile_key<<<nb, BS, 0, stream_>>>(n, tileOf_.as<int>(), lev_.as<int>(), depth_, rs_.as<int>(), lend_.as<int>(),
                                        (unsigned int*)key, val);
     HIPCHK(sortPairs(bits((long long)K * depth_) + kWidthBits));
-    HIPCHK(sorder_.alloc(P4));
-    HIPCHK(pos_.alloc(n4));
-    k_tile_fill_i32<<<blocks(P), BS, 0, stream_>>>(P, -1, sorder_.as<int>());
-    k_tile_place<<<nb, BS, 0, stream_>>>(n, val2, K, S, sorder_.as<int>(), pos_.as<int>());
+    HIPCHK(f_->sorder.alloc(P4));
+    HIPCHK(f_->pos.alloc(n4));
+    k_tile_fill_i32<<<blocks(P), BS, 0, stream_>>>(P, -1, f_->sorder.as<int>());
+    k_tile_place<<<nb, BS, 0, stream_>>>(n, val2, K, S, f_->sorder.as<int>(), f_->pos.as<int>());
     // counts and their prefix sums
     HIPCHK(tileCnt_.alloc(4 * P4 + 2 * (size_t)nch * 4));
-    HIPCHK(tileStep_.alloc((size_t)P));
+    HIPCHK(f_->tileStep.alloc((size_t)P));
     HIPCHK(entryHalo_.alloc((size_t)nnz_ * 4));
     int* eh = entryHalo_.as<int>();
     int* cnt[2][2];
@@ -751,13 +745,13 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
         cnt[d][1] = cnt[d][0] + P;                           // exports
         wid[d] = tileCnt_.as<int>() + 4 * (size_t)P + d * nch;
     }
-    const TilePattern M{P, S, sorder_.as<int>(), pos_.as<int>(), rs_.as<int>(), lend_.as<int>(), ubeg_.as<int>(),
+    const TilePattern M{P, S, f_->sorder.as<int>(), f_->pos.as<int>(), rs_.as<int>(), lend_.as<int>(), ubeg_.as<int>(),
                         col_.as<int>(), tpos_.as<int>(), lev_.as<int>()};
     const int pb = blocks(P);
     k_tile_fill_i32<<<blocks(nnz_), BS, 0, stream_>>>((int)nnz_, 0, eh);
     k_tile_mark<0><<<pb, BS, 0, stream_>>>(M, cnt[0][1], eh);
     k_tile_mark<1><<<pb, BS, 0, stream_>>>(M, cnt[1][1], eh);
-    k_tile_count<<<pb, BS, 0, stream_>>>(M, eh, cnt[0][0], cnt[1][0], tileStep_.as<uint8_t>(), wid[0], wid[1]);
+    k_tile_count<<<pb, BS, 0, stream_>>>(M, eh, cnt[0][0], cnt[1][0], f_->tileStep.as<uint8_t>(), wid[0], wid[1]);
     auto scan = [&](const int* in, DevBuf& out, int m) -> hipError_t {  // out[0] = 0, out[k + 1] = in[0] + .. + in[k]
         size_t tb = 0;
         hipError_t e = out.alloc(((size_t)m + 1) * 4);
@@ -768,20 +762,20 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
         return e;
     };
     for (int d = 0; d < 2; ++d) {
-        HIPCHK(scan(cnt[d][0], tile_[d].hstart, P));
-        HIPCHK(scan(cnt[d][1], tile_[d].xstart, P));
-        HIPCHK(scan(wid[d], tile_[d].sell, nch));
+        HIPCHK(scan(cnt[d][0], f_->tile[d].hstart, P));
+        HIPCHK(scan(cnt[d][1], f_->tile[d].xstart, P));
+        HIPCHK(scan(wid[d], f_->tile[d].sell, nch));
     }
     HIPCHK(tileMax_.alloc(8));
     k_tile_fill_i32<<<1, BS, 0, stream_>>>(2, 0, tileMax_.as<int>());
-    k_tile_max<<<blocks(K), BS, 0, stream_>>>(K, S, tile_[0].hstart.as<int>(), tile_[1].hstart.as<int>(),
-                                              tile_[0].xstart.as<int>(), tile_[1].xstart.as<int>(),
+    k_tile_max<<<blocks(K), BS, 0, stream_>>>(K, S, f_->tile[0].hstart.as<int>(), f_->tile[1].hstart.as<int>(),
+                                              f_->tile[0].xstart.as<int>(), f_->tile[1].xstart.as<int>(),
                                               tileMax_.as<int>());
     HIPCHK(hipGetLastError());
     int* h = reinterpret_cast<int*>(hplan_);
     for (int d = 0; d < 2; ++d) {
-        HIPCHK(hipMemcpyAsync(h + 2 * d, tile_[d].hstart.as<int>() + P, 4, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipMemcpyAsync(h + 2 * d + 1, tile_[d].sell.as<int>() + nch, 4, hipMemcpyDeviceToHost, stream_));
+        HIPCHK(hipMemcpyAsync(h + 2 * d, f_->tile[d].hstart.as<int>() + P, 4, hipMemcpyDeviceToHost, stream_));
+        HIPCHK(hipMemcpyAsync(h + 2 * d + 1, f_->tile[d].sell.as<int>() + nch, 4, hipMemcpyDeviceToHost, stream_));
     }
     HIPCHK(hipMemcpyAsync(h + 4, tileMax_.p, 8, hipMemcpyDeviceToHost, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
@@ -791,14 +785,14 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
                 "%lld %lld\n", n, depth_, K, kk[0], kk[1], kk[2], S, h[4], h[5], (long long)h[1] * 128,
                 (long long)h[3] * 128);
     // slots are named by 16 bits; the values and the export list share the LDS
-    tileExports_ = h[5];
-    if (slots > 65536 || !tilesFit((int)slots, width)) return ASTG_OK;
-    if (!placed && !forced && !rangesPay(depth_, S, h[4])) return ASTG_OK;
-    tileK_ = K;
-    tileS_ = S;
-    tileSlots_ = (int)slots;
+    f_->tileExports = h[5];
+    f_->tileSlots = (int)std::min<long long>(slots, 65537);
+    if (slots > 65536 || !tilesFit(width)) return ASTG_OK;
+    if (!placed && tilesAsked_ < 0 && !rangesPay(depth_, S, h[4])) return ASTG_OK;
+    f_->tileK = K;
+    f_->tileS = S;
     for (int d = 0; d < 2; ++d) {
-        DevTile& D = tile_[d];
+        DevTile& D = f_->tile[d];
         D.E = (long long)h[2 * d + 1] * 128;
         D.halo = h[2 * d];
         // every halo entry is one export of another tile
@@ -815,8 +809,7 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
                                    D.slot.as<uint32_t>());
     }
     HIPCHK(hipGetLastError());
-    PS_ = P;
-    tileLds64_ = tileLds32_ = false;  // the form of the kernel may have changed
+    f_->PS = P;
     used = true;
     return ASTG_OK;
 }
@@ -824,23 +817,23 @@ int PcgDevice::tileSetup(bool& used, std::string& err) {
 TileView PcgDevice::tileView() const {
     TileView v;
     for (int d = 0; d < 2; ++d) {
-        v.d[d].sell = tile_[d].sell.as<int>();
-        v.d[d].slot = tile_[d].slot.as<uint32_t>();
-        v.d[d].hstart = tile_[d].hstart.as<int>();
-        v.d[d].xstart = tile_[d].xstart.as<int>();
-        v.d[d].xslot = tile_[d].xslot.as<uint16_t>();
-        v.d[d].xdest = tile_[d].xdest.as<int>();
+        v.d[d].sell = f_->tile[d].sell.as<int>();
+        v.d[d].slot = f_->tile[d].slot.as<uint32_t>();
+        v.d[d].hstart = f_->tile[d].hstart.as<int>();
+        v.d[d].xstart = f_->tile[d].xstart.as<int>();
+        v.d[d].xslot = f_->tile[d].xslot.as<uint16_t>();
+        v.d[d].xdest = f_->tile[d].xdest.as<int>();
     }
-    v.step = tileStep_.as<uint8_t>();
-    v.order = sorder_.as<int>();
+    v.step = f_->tileStep.as<uint8_t>();
+    v.order = f_->sorder.as<int>();
     // the upper word of each system's B_DONE
     static_assert(kSysStride == 2 * B_COUNT, "state of a system");
-    v.sys = K_ ? tileSys_.as<int>() : nullptr;
+    v.sys = K_ ? f_->tileSys.as<int>() : nullptr;
     v.ndone = K_ ? bcnt_.as<int>() : nullptr;
     v.sysDone = K_ ? bst_.as<int>() + 2 * B_DONE + 1 : nullptr;
-    v.S = tileS_;
-    v.slots = tileSlots_;
-    v.exports = tileExports_;
+    v.S = f_->tileS;
+    v.slots = f_->tileSlots;
+    v.exports = f_->tileExports;
     v.trace = trace_;
     return v;
 }
@@ -850,22 +843,14 @@ bool PcgDevice::isTileKernel(const void* f) const {
            f == (const void*)k_tile_sweep<double, kTileByRow> || f == (const void*)k_tile_sweep<float, kTileByRow>;
 }
 
-// FP64 solves: the coefficients of the current factor, gathered once per factor.
-int PcgDevice::ensureTileCoef64(std::string& err) {
-    if (!tiled_ || tileCoef64_) return ASTG_OK;
-    if (int rc = tileCoef<double>(err)) return rc;
-    tileCoef64_ = true;
-    return ASTG_OK;
-}
-
 template <typename T>
 int PcgDevice::tileCoef(std::string& err) {
     for (int d = 0; d < 2; ++d) {
-        DevBuf& c = sizeof(T) == 8 ? tile_[d].coef : tile_[d].coef32;
-        HIPCHK(c.alloc(std::max<size_t>(16, (size_t)tile_[d].E * sizeof(T))));
+        DevBuf& c = sizeof(T) == 8 ? f_->tile[d].coef : f_->tile[d].coef32;
+        HIPCHK(c.alloc(std::max<size_t>(16, (size_t)f_->tile[d].E * sizeof(T))));
         auto k = d == 0 ? k_tile_coef<T, 0> : k_tile_coef<T, 1>;
-        k<<<blocks(PS_), BS, 0, stream_>>>(PS_, sorder_.as<int>(), rs_.as<int>(), lend_.as<int>(), ubeg_.as<int>(),
-                                           F_.as<double>(), tile_[d].sell.as<int>(), c.as<Pair<T>>());
+        k<<<blocks(f_->PS), BS, 0, stream_>>>(f_->PS, f_->sorder.as<int>(), rs_.as<int>(), lend_.as<int>(), ubeg_.as<int>(),
+                                           F_.as<double>(), f_->tile[d].sell.as<int>(), c.as<Pair<T>>());
     }
     HIPCHK(hipGetLastError());
     return ASTG_OK;
@@ -874,36 +859,37 @@ int PcgDevice::tileCoef(std::string& err) {
 template <typename T>
 int PcgDevice::launchTile(const T* invd, const T* r, T* z, int k, int mode, int it, int maxIt, int norm,
                           double tolRel, int phases, std::string& err) {
-    const auto kernel = !perm_   ? k_tile_sweep<T, kTileByRow>
-                        : trace_ ? k_tile_sweep<T, kTileTrace>
-                                 : k_tile_sweep<T, kTilePlain>;
-    const size_t lds = tileLds(tileSlots_, sizeof(T));
-    bool& raised = sizeof(T) == 8 ? tileLds64_ : tileLds32_;
-    if (!raised || trace_) {
+    const TileMode form = !perm_ ? kTileByRow : trace_ ? kTileTrace : kTilePlain;
+    const auto kernel = form == kTileByRow   ? k_tile_sweep<T, kTileByRow>
+                        : form == kTileTrace ? k_tile_sweep<T, kTileTrace>
+                                             : k_tile_sweep<T, kTilePlain>;
+    const size_t lds = tileLds(sizeof(T));
+    bool& raised = tileLds_[sizeof(T) == 8][form];
+    if (!raised) {
         HIPCHK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)kTileLdsBytes));
         raised = true;
     }
     TileView V = tileView();
-    const Pair<T>* cF = (const Pair<T>*)(sizeof(T) == 8 ? tile_[0].coef.p : tile_[0].coef32.p);
-    const Pair<T>* cB = (const Pair<T>*)(sizeof(T) == 8 ? tile_[1].coef.p : tile_[1].coef32.p);
+    const Pair<T>* cF = (const Pair<T>*)(sizeof(T) == 8 ? f_->tile[0].coef.p : f_->tile[0].coef32.p);
+    const Pair<T>* cB = (const Pair<T>*)(sizeof(T) == 8 ? f_->tile[1].coef.p : f_->tile[1].coef32.p);
     T* y = y_.as<T>();
-    T* xF = tile_[0].inbox.as<T>() + (size_t)(k & 1) * tile_[0].halo;
-    T* nF = tile_[0].inbox.as<T>() + (size_t)((k + 1) & 1) * tile_[0].halo;
-    T* xB = tile_[1].inbox.as<T>() + (size_t)(k & 1) * tile_[1].halo;
-    T* nB = tile_[1].inbox.as<T>() + (size_t)((k + 1) & 1) * tile_[1].halo;
-    Parts Pt = parts(tileK_);
+    T* xF = f_->tile[0].inbox.as<T>() + (size_t)(k & 1) * f_->tile[0].halo;
+    T* nF = f_->tile[0].inbox.as<T>() + (size_t)((k + 1) & 1) * f_->tile[0].halo;
+    T* xB = f_->tile[1].inbox.as<T>() + (size_t)(k & 1) * f_->tile[1].halo;
+    T* nB = f_->tile[1].inbox.as<T>() + (size_t)((k + 1) & 1) * f_->tile[1].halo;
+    Parts Pt = parts(f_->tileK);
     int* cnt = cnt_.as<int>();
     double* scal = scal_.as<double>();
     int parity = k & 1;
     if (!coop_) {
-        kernel<<<tileK_, kTileThreads, lds, stream_>>>(V, cF, cB, invd, r, y, z, xF, xB, nF, nB, Pt, cnt, scal, mode,
+        kernel<<<f_->tileK, kTileThreads, lds, stream_>>>(V, cF, cB, invd, r, y, z, xF, xB, nF, nB, Pt, cnt, scal, mode,
                                                        it, maxIt, norm, tolRel, parity, phases);
         HIPCHK(hipGetLastError());
     } else {
         void* args[] = {&V,  &cF, &cB,  &invd, &r,    &y,    &z,  &xF,    &xB,   &nF,     &nB,
                         &Pt, &cnt, &scal, &mode, &it, &maxIt, &norm, &tolRel, &parity, &phases};
-        HIPCHK(hipLaunchCooperativeKernel((const void*)kernel, dim3(tileK_), dim3(kTileThreads), args,
+        HIPCHK(hipLaunchCooperativeKernel((const void*)kernel, dim3(f_->tileK), dim3(kTileThreads), args,
                                           (unsigned)lds, stream_));
     }
     return ASTG_OK;

@@ -310,3 +310,75 @@ def test_no_tiles_are_set_up_for_rows_that_do_not_fit(tiles, done, monkeypatch, 
     c.close()
     assert r.converged == 1
     assert ("tiles: n 24000 " in capfd.readouterr().err) == done
+
+
+@pytest.fixture
+def narrow(monkeypatch):
+    """A projection in block colours whose tiles hold 20 k to 40 k rows: more
+    than 160 KB in FP64, less in FP32."""
+    from astg import scenes
+    ctx, info = scenes.smoke_64(device=0, R=96)
+    scenes.fill_velocity(ctx, info["levels"], 3)
+    monkeypatch.setenv("ASTG_TILES", str(max(1, round(ctx.numbering(0)[2] / 28000))))
+    ctx.snapshot(False)
+
+    def project(precision, tol=1e-10):
+        import astg
+        prm = astg.default_params(tol=tol, max_iterations=3000, ordering=astg.ORDER_BLOCK_COLOUR,
+                                  precision=astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64)
+        ctx.snapshot(True)
+        r = ctx.project(info["dt"], info["rho"], prm)
+        return r, ctx.system(r.n, r.nnz)[4]
+
+    yield ctx, project
+    ctx.close()
+
+
+def test_each_precision_keeps_its_sweeps(narrow, monkeypatch, capfd):
+    """Mixed and FP64 solves in turn on one pattern: the mixed one stays in
+    tiles, the FP64 one merged, whatever came before, and neither is set up a
+    second time. Which form a solve took shows in its solution's last bits."""
+    monkeypatch.setenv("ASTG_TIMING", "1")
+    ctx, project = narrow
+    m0, f0 = project("mixed"), project("fp64")
+    capfd.readouterr()
+    m1, f1, f2, m2 = project("mixed"), project("fp64"), project("fp64"), project("mixed")
+    assert "timing] sweeps/" not in capfd.readouterr().err
+    for a, b in ((m0, m1), (m0, m2), (f0, f1), (f0, f2)):
+        assert a[0].iterations == b[0].iterations and np.array_equal(a[1], b[1])
+
+
+def test_fp64_projections_set_no_fp32_tiles_up(narrow, monkeypatch, capfd):
+    monkeypatch.setenv("ASTG_TIMING", "1")
+    ctx, project = narrow
+    capfd.readouterr()
+    f0 = project("fp64")
+    err = capfd.readouterr().err
+    assert "tiles: n" not in err and err.count("timing] sweeps/merged order") == 1
+    project("mixed")
+    assert "tiles: n" in capfd.readouterr().err
+    assert np.array_equal(project("fp64")[1], f0[1])
+
+
+@pytest.mark.parametrize("which", ["FWD64", "BWD64"])
+def test_fp64_sweeps_can_be_timed_after_a_mixed_solve(narrow, which):
+    import astg
+    ctx, project = narrow
+    m0 = project("mixed")
+    ms, by = ctx.kernel_time(getattr(astg, "K_" + which), 2)
+    assert ms > 0 and by > 0
+    t, lev = ctx.sweep_timeline(getattr(astg, "K_" + which), m0[0].n)
+    assert (t[:, 2] > 0).all() and lev.min() == 0
+    assert np.array_equal(project("mixed")[1], m0[1])
+
+
+def test_a_mixed_projection_sets_one_systems_sweeps_up(monkeypatch, capfd):
+    """The block-colour copy's: the reference numbering is not swept."""
+    import astg
+    from astg import scenes
+    monkeypatch.setenv("ASTG_TIMING", "1")
+    ctx, info = scenes.smoke_64(device=0)
+    scenes.fill_velocity(ctx, info["levels"], 3)
+    ctx.project(info["dt"], info["rho"], astg.default_params(tol=1e-6, precision=astg.PREC_MIXED))
+    ctx.close()
+    assert capfd.readouterr().err.count("timing] sweeps/permuted pattern") == 1
