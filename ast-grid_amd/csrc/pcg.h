@@ -25,6 +25,7 @@
 
 #include "../../include/astg.h"
 #include "device_common.h"
+#include "sweep_room.h"
 #include "tile_sweep.h"
 
 namespace astg {
@@ -288,6 +289,9 @@ private:
                    const char* what, std::string& err);
     int formVectors(std::string& err);
     int ensureCoef64(std::string& err);
+    // The compute units that the current form's sweeps rely on holding at once.
+    int sweepUnits() const;
+    SweepRoom& sweepRoom() const;  // of this object's device
     // Sweep-ordered solve: permuted CSR, forward r-term keys as positions
     // (once per form); values, pivots and rhs gathered per solve.
     int permuteSetup(std::string& err);
@@ -373,6 +377,7 @@ private:
     int P_ = 0;                             // padded length of the level order
     int merge_ = 2;                         // levels per super-level of the sweeps
     int cus_ = 0;                           // compute units
+    int device_ = 0;
     int gs_ = 0;                            // grid of the streaming kernels
     int gb_ = 0;                            // largest backward-sweep grid (rho partial slots)
     int gateDist_ = 2;                      // sweep gates: groups back (forward) / ahead

@@ -1052,6 +1052,7 @@ int PcgDevice::setPatternImpl(int n, long long nnz, const int* dRowstart, const 
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     cus_ = cus;
+    device_ = dev;
     // streaming kernels: 8 blocks (32 wavefronts) per CU in a grid-stride loop;
     // this many partials is still cheap to reduce in the consumer kernel
     gs_ = std::max(1, std::min(8 * cus, blocks(n)));
@@ -1505,6 +1506,19 @@ int PcgDevice::launchBwd(const T* invd, const T* r, T* z, int k, int parityOut, 
     return ASTG_OK;
 }
 
+// A tile waits for any other tile. Merged sweeps wait for chunks before their
+// own: with a block per chunk those are resident or done, with fewer blocks than
+// chunks the whole grid (at the occupancy limit) has to be.
+int PcgDevice::sweepUnits() const {
+    if (f_->tiled) return f_->tileK;
+    const int grid = std::min({f_->gF64, f_->gF32, f_->gB64, f_->gB32});
+    return f_->PS / BS > grid ? cus_ : 0;
+}
+SweepRoom& PcgDevice::sweepRoom() const {
+    static SweepRoom rooms[64];
+    return rooms[device_ & 63];
+}
+
 // The values that the first sweep of a solve waits for.
 template <typename T>
 void PcgDevice::armSweeps() {
@@ -1603,6 +1617,7 @@ int PcgDevice::solveOnce(const astg_pcg_params& prm, astg_pcg_result& res, std::
     if (int rc = useForm(prm.precision, err)) return rc;
     if (prm.precision == ASTG_PREC_FP64)
         if (int rc = ensureCoef64(err)) return rc;
+    const SweepLease lease(sweepRoom(), sweepUnits(), cus_);
     const int n = vlen(), gs = gs_;
     res.n = n_;
     res.nnz = nnz_;
@@ -1732,6 +1747,7 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
     if (f32 || sweep64s || !f_->ready) {
         if (int rc = useForm(f32 ? ASTG_PREC_MIXED : ASTG_PREC_FP64, err)) return rc;
     }
+    const SweepLease lease(sweepRoom(), sweepUnits(), cus_);
     const int nv = vlen();
     // the solve's own layout: sweep-ordered vectors and CSR unless the row order is kept
     if (int rc = prepareSolve(err)) return rc;

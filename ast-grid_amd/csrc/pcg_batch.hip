@@ -506,6 +506,7 @@ int PcgDevice::solveBatchOnce(const astg_pcg_params& prm, std::vector<astg_pcg_r
         return ASTG_ERR_ARG;
     }
     if (int rc = useForm(prm.precision, err)) return rc;
+    const SweepLease lease(sweepRoom(), sweepUnits(), cus_);
     const BatchView V = bview();
     const int g = batchGrid();
     const int maxIt = std::max(0, prm.max_iterations);

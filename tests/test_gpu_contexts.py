@@ -58,3 +58,63 @@ def test_interleaved_contexts_match_single_runs():
             assert np.array_equal(x, y)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_solves_of_two_threads_leave_each_other_room(precision, monkeypatch, capfd):
+    """Two contexts, a thread and a stream each, whose sweeps rely on 180 and
+    120 compute units: together more than the device has. No sweep waits for a
+    workgroup that found no room (which would be reported and retried), and the
+    results are those of a context alone; a third one, small enough to fit
+    beside either, runs along."""
+    import threading
+
+    import astg
+    from astg import scenes
+    prm = astg.default_params(tol=1e-9, max_iterations=3000,
+                              precision=astg.PREC_MIXED if precision == "mixed" else astg.PREC_FP64)
+    g = load_golden("%s/tests/golden/s16_sphere.npz" % ROOT)
+    system = (g["A_rowstart"], g["A_col"], g["A_val"], g["b"])
+
+    def octree(tiles):
+        # both threads' contexts are made, and solve once, before they start
+        monkeypatch.setenv("ASTG_TILES", str(tiles))
+        ctx, info = scenes.smoke_64(device=0)
+        scenes.fill_velocity(ctx, info["levels"], 3)
+        ctx.snapshot(False)
+
+        def go():
+            ctx.snapshot(True)
+            r = ctx.project(info["dt"], info["rho"], prm)
+            return ctx.system(r.n, r.nnz)[4]
+        return ctx, go
+
+    def seam():
+        monkeypatch.delenv("ASTG_TILES")
+        ctx = astg.Context(0)
+
+        def go():
+            return ctx.pcg_solve_csr(*system, prm)[0]
+        return ctx, go
+
+    made = [octree(200), octree(128), seam()]
+    want = [go() for _, go in made]
+    wrong = []
+
+    def work(go, x):
+        try:
+            for _ in range(12):
+                if not np.array_equal(go(), x):
+                    wrong.append("another result")
+        except Exception as e:  # noqa: BLE001 (reported below)
+            wrong.append(e)
+
+    threads = [threading.Thread(target=work, args=(go, x)) for (_, go), x in zip(made, want)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for ctx, _ in made:
+        ctx.close()
+    assert not wrong
+    assert "retrying" not in capfd.readouterr().err
