@@ -165,6 +165,8 @@ struct BatchView {
     double* part;         // one partial per chunk
     int* ndone;           // systems finished in the current inner solve
     int K, nchunks;
+    int* tileFin;         // per tile of the sweeps: nonzero once a system with rows in it has finished
+    int tiles;            // 0: merged sweeps
 };
 
 class PcgDevice {
@@ -386,6 +388,7 @@ private:
     long long* trace_ = nullptr;            // set only while a timeline is recorded
     int K_ = 0;                             // batched form: systems in the stack (0: single system)
     DevBuf chunkSeg_, segChunk_, bst_, bpart_, bcnt_;  // batched form: layout, state, partials, counter
+    DevBuf tileFin_;                        // batched form: BatchView::tileFin
     int blocksPerCu_ = 0;                   // batched form: streaming grid (0: gs_)
     int lpr_ = 8;                           // batched form: SpMV lanes per row
     int mergeLevels_ = 0;                   // requested levels per sweep group (0: default)

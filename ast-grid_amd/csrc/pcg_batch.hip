@@ -54,6 +54,17 @@ __global__ void __launch_bounds__(BS) kb_init(BatchView V, const T* b, X* x, T* 
     }
 }
 
+// System k has finished: its tiles (row i is in tile i * tiles / rows) are
+// marked, and the last system to finish ends the sweeps. One thread.
+__device__ inline void finish(const BatchView& V, int k, double* scal) {
+    if (V.tiles) {
+        const long long n = (long long)V.nchunks * BS, r0 = (long long)V.segChunk[k] * BS,
+                        r1 = (long long)V.segChunk[k + 1] * BS - 1;
+        for (int b = (int)(r0 * V.tiles / n); b <= (int)(r1 * V.tiles / n); ++b) V.tileFin[b] = 1;
+    }
+    if (atomicAdd(V.ndone, 1) + 1 == V.K) scal[S_DONE] = 1.0;
+}
+
 // One block per system: the system's partials in chunk order, then the
 // phase's scalar update (thread 0). A system that finishes here is counted;
 // the last one to finish raises the all-done flag that ends the sweeps.
@@ -74,7 +85,7 @@ __global__ void __launch_bounds__(BS) kb_reduce(BatchView V, int phase, int norm
         s[B_RES] = red;  // a NaN or infinity in this system's b or residual: it stops (state 5)
         if (phase == P_RES) s[B_ITER] += 1.0;
         s[B_DONE] = 5.0;
-        if (atomicAdd(V.ndone, 1) + 1 == V.K) scal[S_DONE] = 1.0;
+        finish(V, k, scal);
         return;
     }
     switch (phase) {
@@ -129,7 +140,7 @@ __global__ void __launch_bounds__(BS) kb_reduce(BatchView V, int phase, int norm
             s[B_OUTER] = red;
             break;
     }
-    if (fin && atomicAdd(V.ndone, 1) + 1 == V.K) scal[S_DONE] = 1.0;
+    if (fin) finish(V, k, scal);
 }
 
 // Partials of z.r per chunk (the single-system form fuses this dot into the
@@ -264,7 +275,8 @@ __global__ void __launch_bounds__(BS) kb_add_corr(BatchView V, double* x, const 
     }
 }
 
-__global__ void kb_zero_count(int* c) {
+__global__ void kb_zero_count(int* c, int* tileFin, int tiles) {
+    for (int b = threadIdx.x; b < tiles; b += blockDim.x) tileFin[b] = 0;
     if (threadIdx.x == 0) c[0] = 0;
 }
 __global__ void kb_zero64(int n, double* x) {
@@ -325,6 +337,8 @@ BatchView PcgDevice::bview() const {
     v.ndone = bcnt_.as<int>();
     v.K = K_;
     v.nchunks = n_ / BS;
+    v.tileFin = tileFin_.as<int>();
+    v.tiles = f_->tiled ? f_->tileK : 0;
     return v;
 }
 
@@ -367,7 +381,7 @@ int PcgDevice::pcgBatchInner(const T* A, const T* invd, const T* b, double* x, i
     double* scal = scal_.as<double>();
     int rc;
     kb_zero64<<<1, BS, 0, stream_>>>(32, scal);
-    kb_zero_count<<<1, 64, 0, stream_>>>(V.ndone);
+    kb_zero_count<<<1, 64, 0, stream_>>>(V.ndone, V.tileFin, V.tiles);
     kb_init<T, double><<<g, BS, 0, stream_>>>(V, b, x, r, norm);
     kb_reduce<<<V.K, BS, 0, stream_>>>(V, P_INIT, norm, scal);
     armSweeps<T>();

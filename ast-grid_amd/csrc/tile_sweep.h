@@ -55,7 +55,7 @@ struct TileView {
     const int* order;  // per position: row, -1 padding
     const int* sys;    // batched solves, per position: the row's system
     const int* sysDone;  // and per system, kSysStride apart: nonzero once it has finished
-    const int* ndone;    // and the number of systems that have
+    const int* finished; // per tile: nonzero once a system with rows in it has
     int S;             // positions per tile
     int slots;         // LDS slots: S + H + 1
     int exports;       // room of the LDS export list

@@ -364,7 +364,7 @@ struct TileChunk {
 };
 template <typename T, int DIR, int MODE>
 __device__ inline void tile_load(TileChunk<T>& C, const TileView& V, const Pair<T>* coef, const T* invd, const T* r,
-                                 const T* y, int chunk, int base, int w) {
+                                 const T* y, int chunk, int base, int w, bool some) {
     const int lane = threadIdx.x & 63;
     C.w = w;
     C.t = chunk * 64 + lane;
@@ -377,7 +377,6 @@ __device__ inline void tile_load(TileChunk<T>& C, const TileView& V, const Pair<
         }
     if constexpr (MODE == kTileByRow) {
         C.v = V.order[C.t];
-        const bool some = *V.ndone != 0;  // changes between launches only
         const int s = some ? V.sys[C.t] : 0;
         C.r = C.inv = (T)0;  // padding: the row's value is zero
         C.done = 0;
@@ -465,10 +464,11 @@ __device__ inline bool tile_rows(const TileChunk<T>& C, T* lds, T* own, T& v, lo
 // One direction over a wavefront's chunks: of the tile's, in level order (DIR 1:
 // reversed), every kTileWaves-th from the wavefront's own, so that a chunk's
 // data is loaded while the chunks before it are worked on. out: y or z; dot: the
-// backward sweep's z.r.
+// backward sweep's z.r; some: a system with rows in the tile has finished.
 template <typename T, int DIR, int MODE>
 __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const T* invd, const T* r, const T* y,
-                                   T* out, double& dot, int p0, int wave, T* lds, long long t0, int* err, int bit) {
+                                   T* out, double& dot, int p0, int wave, T* lds, long long t0, int* err, int bit,
+                                   bool some) {
     const int chunks = V.S / 64, first = p0 / 64 + wave, count = (chunks - wave + kTileWaves - 1) / kTileWaves;
     if (count <= 0) return;
     const int zero = V.slots - 1;
@@ -481,7 +481,7 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
     auto load = [&](TileChunk<T>& C, int j) {
         const int base = j < 64 ? __builtin_amdgcn_readlane(s0, j) : __builtin_amdgcn_readlane(s1, j - 64);
         const int end = j < 64 ? __builtin_amdgcn_readlane(e0, j) : __builtin_amdgcn_readlane(e1, j - 64);
-        tile_load<T, DIR, MODE>(C, V, coef, invd, r, y, chunk(j), base, end - base);
+        tile_load<T, DIR, MODE>(C, V, coef, invd, r, y, chunk(j), base, end - base, some);
     };
     auto work = [&](TileChunk<T>& C) {
         if constexpr (MODE == kTileByRow) {
@@ -577,6 +577,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const P
     T* lds = reinterpret_cast<T*>(tile_lds);
     int* xdest = reinterpret_cast<int*>(lds + V.slots);
     uint16_t* xslot = reinterpret_cast<uint16_t*>(xdest + V.exports);
+    const bool some = MODE == kTileByRow && V.finished[blockIdx.x] != 0;  // changes between launches only
     if (sweep_stopped(scal, cnt)) return;
     const int S = V.S, p0 = blockIdx.x * S, zero = V.slots - 1;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -599,7 +600,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const P
         __syncthreads();
         const long long t0 = wall_clock64();
         if (wave < kTileWaves)
-            tile_chunks<T, 0, MODE>(V, coefF, invd, r, y, y, dot, p0, wave, lds, t0, err, E_FWD);
+            tile_chunks<T, 0, MODE>(V, coefF, invd, r, y, y, dot, p0, wave, lds, t0, err, E_FWD, some);
         else if (wave < kTileWaves + kTileImport)
             tile_import<T, 0>(V.d[0], p0, S, xF, lds + S, threadIdx.x - kTileWaves * 64, t0, err, E_FWD);
         else
@@ -612,7 +613,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const P
     __syncthreads();
     const long long t0 = wall_clock64();
     if (wave < kTileWaves)
-        tile_chunks<T, 1, MODE>(V, coefB, invd, r, y, z, dot, p0, wave, lds, t0, err, E_BWD);
+        tile_chunks<T, 1, MODE>(V, coefB, invd, r, y, z, dot, p0, wave, lds, t0, err, E_BWD, some);
     else if (wave < kTileWaves + kTileImport)
         tile_import<T, 1>(V.d[1], p0, S, xB, lds + S, threadIdx.x - kTileWaves * 64, t0, err, E_BWD);
     else
@@ -653,6 +654,7 @@ static __global__ void k_tile_sys(int P, const int* order, const int* chunkSeg, 
 }
 int PcgDevice::tileSystems(std::string& err) {
     HIPCHK(f_->tileSys.alloc((size_t)f_->PS * 4));
+    HIPCHK(tileFin_.alloc((size_t)f_->tileK * 4));
     k_tile_sys<<<blocks(f_->PS), BS, 0, stream_>>>(f_->PS, f_->sorder.as<int>(), chunkSeg_.as<int>(), f_->tileSys.as<int>());
     HIPCHK(hipGetLastError());
     return ASTG_OK;
@@ -829,7 +831,7 @@ TileView PcgDevice::tileView() const {
     // the upper word of each system's B_DONE
     static_assert(kSysStride == 2 * B_COUNT, "state of a system");
     v.sys = K_ ? f_->tileSys.as<int>() : nullptr;
-    v.ndone = K_ ? bcnt_.as<int>() : nullptr;
+    v.finished = K_ ? tileFin_.as<int>() : nullptr;
     v.sysDone = K_ ? bst_.as<int>() + 2 * B_DONE + 1 : nullptr;
     v.S = f_->tileS;
     v.slots = f_->tileSlots;
