@@ -3,27 +3,31 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
-#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 
 #include "pcg.h"
 #include "pcg_common.h"
 #include "sweep_merge.h"
+#include "tile_grid.h"
 #include "tile_sweep.h"
 
 namespace astg {
 
 namespace {
 
-// Rows per tile. With positions: 2048. Fewer rows a tile mean more boundary
-// crossings on the dependency chain, more rows a longer queue of chunks per
-// wavefront; measured flat between about 1300 and 2400 (FP64 forward / backward
-// us: n = 63 k, 27 tiles 41 / 43, 48 tiles 40 / 43, 8 tiles 55 / 58; n = 456 k,
-// 252 tiles 73 / 79, 64 tiles 92 / 94). Without, the tiles are index ranges,
-// whose boundary a grid's chain crosses once per tile, so as few as the LDS
-// holds (n = 152 k, ms per solve: 16 tiles 8.5, 32 10.1, 64 12.9, 128 13.4;
-// merged sweeps 15.3).
+// Rows per tile. With positions: about 2048 asked for, before the boxes' shape
+// is chosen (tile_grid.h). Fewer rows a tile mean more boundary crossings on the
+// dependency chain, more rows a longer queue of chunks per wavefront; measured
+// flat between about 1300 and 2400 (FP64 forward / backward us: n = 63 k, 27
+// tiles 41 / 43, 48 tiles 40 / 43, 8 tiles 55 / 58; n = 456 k, 252 tiles 73 / 79,
+// 64 tiles 92 / 94). Without, the tiles are index ranges, whose boundary a
+// grid's chain crosses once per tile, so as few as the LDS holds (n = 152 k, ms
+// per solve: 16 tiles 8.5, 32 10.1, 64 12.9, 128 13.4, merged sweeps 15.3; other
+// sizes, us per FP64 iteration at the tiles that this gives, at fewer and more,
+// and merged: 28^3 3 tiles 80, 2 86, 5 79, merged 162; 36^3 5 tiles 99, 3 114,
+// 8 99, merged 201; 150^2 3 tiles 146, 2 140, 8 160, merged 472; 400^2 17 tiles
+// 378, 9 354, 34 424, merged 1232; 61^3 24 tiles 183, 32 200, merged 336).
 constexpr int kTileRows = 2048;
 constexpr int kTileRangeRows = 9600;
 
@@ -623,25 +627,6 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_sweep(TileView V, const P
     if (threadIdx.x == 0) (parityOut ? Pt.rho1 : Pt.rho0)[blockIdx.x] = s;
 }
 
-// Tile grid: boxes of near-equal edge over the coordinate extents.
-void tileGrid(int K, const int* ext, int* k) {
-    double vol = 1.0;
-    int dims = 0;
-    for (int a = 0; a < 3; ++a)
-        if (ext[a] > 1) {
-            vol *= ext[a];
-            ++dims;
-        }
-    const double edge = dims ? std::pow(vol / K, 1.0 / dims) : 1.0;
-    for (int a = 0; a < 3; ++a) k[a] = ext[a] > 1 ? std::max(1, (int)std::lround(ext[a] / edge)) : 1;
-    while ((long)k[0] * k[1] * k[2] > K) {
-        int m = 0;
-        for (int a = 1; a < 3; ++a)
-            if (k[a] > k[m]) m = a;
-        --k[m];
-    }
-}
-
 }  // namespace
 
 bool PcgDevice::tilesFit(int width) const { return tileLds(width) <= kTileLdsBytes; }
@@ -673,14 +658,17 @@ int PcgDevice::tileSetup(int width, bool& used, std::string& err) {
     const int n = n_;
     const bool placed = coordExt_[0] > 0 && coordN_ == n;
     // a batch's chains end at its systems' boundaries, so its ranges are half as long
-    // (6 systems of 12^3 to 56^3, FP32, ms per solve: 12 tiles 10.7, 16 9.7, 24 9.2, 48 9.6)
+    // (6 systems of 12^3 to 56^3, FP32, ms per solve: 12 tiles 10.7, 16 9.7, 24 9.2, 48 9.6;
+    // other batches, us per FP64 iteration at the tiles that this gives, at fewer and more:
+    // 24 x 20^3 41 tiles 106, 21 129, 82 99; 2 x 30^3 12 tiles 112, 6 133, 24 117; 8 x 40^3
+    // 107 tiles 171, 54 199, 214 185)
     const int range = rowOrderForced_ ? kTileRangeRows / 2 : kTileRangeRows;
     int K = std::min(cus_, placed ? std::max(1, n / kTileRows) : (n + range - 1) / range);
     if (tilesAsked_ == 0) return ASTG_OK;
     if (tilesAsked_ > 0) K = std::min(tilesAsked_, cus_);
     int kk[3] = {1, 1, K};  // tiles per axis
     if (placed) {
-        tileGrid(K, coordExt_, kk);
+        tileGrid(K, n, cus_, coordExt_, kk);
         K = kk[0] * kk[1] * kk[2];
     }
     if (K > n) return ASTG_OK;
