@@ -1154,13 +1154,13 @@ int stackBatch(astg_ctx* c, int count, const int* n, const int* const* rowstart,
 }
 
 // Pattern-only set-up of the stacked system with `merge` levels per sweep
-// group, skipped when the cached pattern is the same.
+// group (which tiles do not have), skipped when the cached pattern is the same.
 int batchPattern(astg_ctx* c, const StackedBatch& S, int merge, bool cache) {
     if (!c->batch) {
         c->batch.reset(new astg::PcgDevice(c->stream));
         c->batch->setRowOrder(true);  // per-system streaming kernels work on stacked rows
     }
-    if (c->batchMerge == merge && c->batchSeg == S.seg && c->batchRs == S.rs && c->batchCol == S.col)
+    if ((c->batchMerge == merge || (c->batchMerge > 0 && c->batch->tiled())) && c->batchSeg == S.seg && c->batchRs == S.rs && c->batchCol == S.col)
         return ASTG_OK;
     c->batchRs.clear();
     c->batchCol.clear();
@@ -1287,7 +1287,7 @@ int astg_pcg_tune_batch(astg_ctx* c, int count, const int* n, const int* const* 
         StackedBatch S;
         int r = stackBatch(c, count, n, rowstart, colindex, value, b, S);
         if (r) return r;
-        static const int kMerge[] = {1, 2, 3};
+        static const int kMerge[] = {2, 1, 3};
         static const int kBlocks[] = {4, 8, 16};
         static const int kLanes[] = {4, 8, 16};
         astg_batch_tuning t;
@@ -1312,6 +1312,7 @@ int astg_pcg_tune_batch(astg_ctx* c, int count, const int* n, const int* const* 
                         t.lanes_per_row = ln;
                     }
                 }
+            if (c->batch->tiled()) break;  // the other values would be the same sweeps
         }
         t.ms_per_iteration = bestMs / iterations;
         c->batchTune = t;

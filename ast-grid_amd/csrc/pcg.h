@@ -242,6 +242,9 @@ public:
     // Levels per merged sweep group used by the next setPattern (0: default).
     void setMergeLevels(int q) { mergeLevels_ = q; }
     int mergeLevels() const { return merge_; }
+    // The current form's sweeps are tiles (known from a pattern's first solve on):
+    // the levels per group do not matter then.
+    bool tiled() const { return f_->ready && f_->tiled; }
     // Solves every system of the stack with its own PCG scalars, convergence
     // test and iteration count (rhs(), solution(), values() hold the stack).
     int solveBatch(const astg_pcg_params& prm, std::vector<astg_pcg_result>& res, std::string& err);

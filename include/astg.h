@@ -147,7 +147,8 @@ int astg_pcg_solve_batch(astg_ctx* ctx, int count, const int* n, const int* cons
 
 /* Launch shape of batched solves (no counterpart in the reference). */
 typedef struct astg_batch_tuning {
-    int merge_levels;         /* dependency levels per merged sweep group, 1-8 (default 2) */
+    int merge_levels;         /* dependency levels per merged sweep group, 1-8 (default 2); a batch
+                               * that sweeps in tiles has no groups and ignores it */
     int stream_blocks_per_cu; /* grid of the streaming kernels, blocks per compute unit, 1-64 (default 8) */
     int lanes_per_row;        /* SpMV lanes per row: 4, 8 (default) or 16 */
     double ms_per_iteration;  /* astg_pcg_tune_batch: one iteration of the chosen shape, ms */
@@ -156,10 +157,10 @@ void astg_batch_tuning_default(astg_batch_tuning* t);
 /* Sets the shape used by the context's next astg_pcg_solve_batch calls. */
 int astg_pcg_set_batch_tuning(astg_ctx* ctx, const astg_batch_tuning* t);
 /* Autotuner: times `iterations` PCG iterations (params' precision; no system
- * converges) of the given batch for merge_levels in {1,2,3} x blocks per CU
- * in {4,8,16} x lanes per row in {4,8,16}, best of two runs each, then sets
- * the fastest shape on the context and returns it in *best. Results of the
- * solves are discarded. */
+ * converges) of the given batch for merge_levels in {1,2,3} (the default only
+ * where the batch sweeps in tiles) x blocks per CU in {4,8,16} x lanes per row
+ * in {4,8,16}, best of two runs each, then sets the fastest shape on the context
+ * and returns it in *best. Results of the solves are discarded. */
 int astg_pcg_tune_batch(astg_ctx* ctx, int count, const int* n, const int* const* rowstart,
                         const int* const* colindex, const double* const* value, const double* const* b,
                         const astg_pcg_params* params, int iterations, astg_batch_tuning* best);

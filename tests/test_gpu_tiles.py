@@ -386,3 +386,30 @@ def test_a_mixed_projection_sets_one_systems_sweeps_up(monkeypatch, capfd):
     ctx.project(info["dt"], info["rho"], astg.default_params(tol=1e-6, precision=astg.PREC_MIXED))
     ctx.close()
     assert capfd.readouterr().err.count("timing] sweeps/permuted pattern") == 1
+
+
+@pytest.mark.parametrize("tiles,patterns", [(3, 2), (0, 4)])
+def test_tuner_times_what_differs(tiles, patterns, monkeypatch, capfd):
+    """In tiles the levels per group are nothing to choose: one pattern is
+    timed (and the chosen one set up), and another value of it takes no new
+    pattern. Merged sweeps are timed with each value."""
+    import astg
+    rng = np.random.default_rng(12)
+    systems = []
+    for shape in ((9, 8, 7), (16, 17, 18)):
+        rs, col, val = box(shape, rng)
+        systems.append((rs, col, val, rng.standard_normal(len(rs) - 1)))
+    monkeypatch.setenv("ASTG_TILES", str(tiles))
+    monkeypatch.setenv("ASTG_TIMING", "1")
+    prm = astg.default_params(tol=1e-8, max_iterations=3000)
+    c = astg.Context(0)
+    best = c.tune_batch(systems, prm, iterations=3)
+    assert capfd.readouterr().err.count("timing] setPattern/factorisation plan") == patterns
+    assert best.merge_levels == 2 or not tiles
+    x, r = c.pcg_solve_batch(systems, prm)
+    c.set_batch_tuning(5, best.stream_blocks_per_cu, best.lanes_per_row)
+    y, q = c.pcg_solve_batch(systems, prm)
+    assert capfd.readouterr().err.count("timing] setPattern/factorisation plan") == (0 if tiles else 1)
+    c.close()
+    for u, v in zip(x, y):
+        assert np.array_equal(u, v) if tiles else np.abs(u - v).max() <= 1e-6 * np.abs(u).max()
