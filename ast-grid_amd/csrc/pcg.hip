@@ -1785,10 +1785,12 @@ int PcgDevice::benchKernel(int which, int reps, double& avgMs, double& bytes, st
             break;
         case ASTG_K_FWD64: case ASTG_K_FWD32: case ASTG_K_BWD64: case ASTG_K_BWD32:
             if (f_->tiled) {
-                // coefficients + slots of the stored entries; per position: r or y, pivot, y or z
-                // written, gate, flag (backward also r for the dot); per halo entry: source, value
+                // coefficients + slots of the stored entries, padding included; per position: r or
+                // y, pivot, y or z written, step (backward also r for the dot); per halo entry: the
+                // value stored and loaded, the next sweep's armed, the export's slot and place
                 const bool bw = which == ASTG_K_BWD64 || which == ASTG_K_BWD32;
-                bytes = (w + 2) * f_->tile[bw ? 1 : 0].E + ((bw ? 4.0 : 3.0) * w + 3) * f_->PS;
+                const DevTile& D = f_->tile[bw ? 1 : 0];
+                bytes = (w + 2) * D.E + ((bw ? 4.0 : 3.0) * w + 1) * f_->PS + (3 * w + 6) * D.halo;
                 break;
             }
             if (which == ASTG_K_BWD64 || which == ASTG_K_BWD32) {

@@ -476,15 +476,15 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
     const int chunks = V.S / 64, first = p0 / 64 + wave, count = (chunks - wave + kTileWaves - 1) / kTileWaves;
     if (count <= 0) return;
     const int zero = V.slots - 1;
-    // the chunks' entry starts and ends, in the lanes of four registers (count <= 128)
+    // the chunks' entry starts and ends, in the lanes of two registers
+    static_assert(kTileLdsBytes / sizeof(float) / 64 / kTileWaves < 64, "chunks of a wavefront");
     const int lane = threadIdx.x & 63;
     auto chunk = [&](int j) { return first + kTileWaves * (DIR == 0 ? j : count - 1 - j); };
-    const int c0 = chunk(min(lane, count - 1)), c1 = chunk(min(lane + 64, count - 1));
+    const int c0 = chunk(min(lane, count - 1));
     const int* sell = V.d[DIR].sell;
-    const int s0 = sell[c0], s1 = sell[c1], e0 = sell[c0 + 1], e1 = sell[c1 + 1];
+    const int s0 = sell[c0], e0 = sell[c0 + 1];
     auto load = [&](TileChunk<T>& C, int j) {
-        const int base = j < 64 ? __builtin_amdgcn_readlane(s0, j) : __builtin_amdgcn_readlane(s1, j - 64);
-        const int end = j < 64 ? __builtin_amdgcn_readlane(e0, j) : __builtin_amdgcn_readlane(e1, j - 64);
+        const int base = __builtin_amdgcn_readlane(s0, j), end = __builtin_amdgcn_readlane(e0, j);
         tile_load<T, DIR, MODE>(C, V, coef, invd, r, y, chunk(j), base, end - base, some);
     };
     auto work = [&](TileChunk<T>& C) {

@@ -18,6 +18,14 @@ from conftest import GOLDEN, load_golden, make_context
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(params=["tiled", "merged"])
+def sweeps(request, monkeypatch):
+    """These systems sweep in tiles by themselves, where only the factorisation
+    plan and order are compared; merged sweeps have the stencils and their order."""
+    if request.param == "merged":
+        monkeypatch.setenv("ASTG_TILES", "0")
+
+
 def _project(g, precision):
     import astg
     c = make_context(g, 0)
@@ -50,7 +58,7 @@ def _same_arrays(a, b):
 
 
 @pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
-def test_projection_identical_with_host_plans(golden, precision, monkeypatch):
+def test_projection_identical_with_host_plans(golden, precision, sweeps, monkeypatch):
     host, dev = _both(monkeypatch, lambda: _project(golden, precision))
     assert host["iters"] == dev["iters"]
     assert host["res"] == dev["res"]
@@ -59,7 +67,7 @@ def test_projection_identical_with_host_plans(golden, precision, monkeypatch):
     assert _same_arrays(host["vel"], dev["vel"])
 
 
-def test_batched_solve_identical_with_host_plans(monkeypatch):
+def test_batched_solve_identical_with_host_plans(sweeps, monkeypatch):
     import astg
     gs = [load_golden(p) for p in GOLDEN]
     systems = [(g["A_rowstart"], g["A_col"], g["A_val"], g["b"]) for g in gs]
@@ -76,7 +84,7 @@ def test_batched_solve_identical_with_host_plans(monkeypatch):
     assert _same_arrays(xh, xd)
 
 
-def test_adaptive_smoke_steps_identical_with_host_plans(monkeypatch):
+def test_adaptive_smoke_steps_identical_with_host_plans(sweeps, monkeypatch):
     import astg
     from astg import scenes
     prm = astg.default_params(tol=1e-6, max_iterations=3000)
