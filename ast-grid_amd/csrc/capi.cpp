@@ -531,7 +531,7 @@ double micTau(const astg_pcg_params& prm) {
 
 // ASTG_ORDER_AUTO: the block-colour form for the mixed precision, the
 // reference numbering for FP64. The block-colour copy is built on the device
-// (C2: 26 ms against a 58 ms solve), so it pays from the first solve on a
+// (C2: 29 ms, its tiles included, against a 55 ms projection), so it pays from the first solve on a
 // pattern, also in a run whose tilts change every step.
 bool blockOrdered(const astg_pcg_params& prm) {
     if (prm.ordering == ASTG_ORDER_BLOCK_COLOUR) return true;

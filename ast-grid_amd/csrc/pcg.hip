@@ -1,6 +1,6 @@
 // Device MIC(0)-PCG (see pcg.h). Kernels are written for gfx950 wave64.
 //
-// Synchronisation design
+// Synchronisation design (of the merged sweeps; the tiled ones: tile_sweep.h)
 //   * The sweeps process rows in order of groups of q consecutive dependency
 //     levels, every group padded so a 64-row wavefront segment holds rows of
 //     one group only. Within a group, rows depend only on earlier groups

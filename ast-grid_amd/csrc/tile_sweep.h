@@ -17,13 +17,13 @@
 // then padding (empty rows). The tile's wavefronts take 64-row chunks in turn.
 // A chunk's entries are stored in pairs, pair by pair (64 lanes side by side),
 // padded to the chunk's widest row (a level's rows are sorted by their lower
-// entries, so forward 30 % and backward 55 % of the entries are padding in an
+// entries, so forward 31 % and backward 56 % of the entries are padding in an
 // octree of 3.5 M rows in block colours). An entry names the LDS slot of its
 // value: [0, S) the tile's rows, [S, S + H) values imported from other tiles
 // ("halo"), S + H a slot that always holds zero (padding entries). A tile's halo
-// entries lie side by side in
-// memory, in the order its rows need them; the tile that computes a value
-// stores it there, once per reading tile, so polling reads whole cache lines.
+// entries lie side by side in memory, in the order its rows need them; the tile
+// that computes a value stores it there, once per reading tile, so polling reads
+// whole cache lines.
 #pragma once
 
 #include <cstdint>
