@@ -617,6 +617,7 @@ int AstUniform::project(double dt, double rho, const astg_pcg_params& prmIn, ast
     (void)hipEventRecord(ev_[0], stream_);
     int rc = ensurePattern(err);
     if (rc) return rc;
+    if (!blocks && (rc = pcg_.prepareSweeps(prmIn.precision, err))) return rc;
     const int n = n_;
     MacPtrs m{{mac_[0].as<double>(), mac_[1].as<double>(), g_.d == 3 ? mac_[2].as<double>() : nullptr}};
     const double scale = rho / dt;
@@ -660,6 +661,7 @@ int AstUniform::project(double dt, double rho, const astg_pcg_params& prmIn, ast
         if (blocks) {
             if ((rc = ensureBlockOrder(err))) return rc;
             S = pcgBlk_.get();
+            if ((rc = S->prepareSweeps(prm.precision, err))) return rc;
             if ((rc = gatherPermuted(stream_, nnz_, blk_.src.as<int>(), pcg_.values(), S->values(), n,
                                      blk_.perm.as<int>(), pcg_.rhs(), S->rhs(), err)))
                 return rc;

