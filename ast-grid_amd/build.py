@@ -24,6 +24,10 @@ SOURCES = ["octree.cpp", "scene.cpp", "weights.cpp", "project_host.cpp", "capi.c
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # host loops at 32-byte boundaries: where the link happened to put the node-set
+    # loops decided a quarter of their time (256^3 topology 400 or 500 ms, the same
+    # object code at two addresses)
+    "-Xarch_host", "-falign-loops=32",
     "-Wall", "-Wno-unused-result", "-I" + os.path.join(HERE, "..", "include"),
 ]
 
