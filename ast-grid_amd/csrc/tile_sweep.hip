@@ -568,7 +568,8 @@ __device__ inline void tile_chunks(const TileView& V, const Pair<T>* coef, const
 // holds by the stream of coefficients. Measured us, forward / backward, merged
 // sweeps before and tiles now: FP64 reference order n = 63 k (71 levels) 69 / 89
 // and 41 / 43, 456 k (133) 140 / 175 and 73 / 79; FP32 block colours 198 k (61)
-// 108 / 104 and 46 / 47, 3.5 M (67) 144 / 147 and 77 / 92.
+// 108 / 104 and 46 / 47, 3.5 M (67) 144 / 147 and 65 / 80 (FP64, 262 levels,
+// 312 / 381 and 213 / 238).
 // xF / xB: the halo entries of this sweep (armed by the sweep before), nF / nB:
 // those of the next one, armed here. A position is worked on by the
 // same lane in both sweeps, so y needs no hand-over.
